@@ -659,4 +659,28 @@ hipError_t dgemm_mfma_batched(int M, int N, int K, double alpha, const double* A
   }
 }
 
+// Grams of consecutive column blocks of V in one launch: block b (w columns at
+// V + b w ldv, n rows) split over the rows into ns slices of kslice, the raw
+// slices at part + (b ns + z) ldp^2 (w x w, leading dimension ldp).  64 x 64
+// tiles: the blocks are few and the slices are what fills the chip.
+hipError_t dgemm_gram_batched(int n, int w, int ldp, const double* V, long ldv, int kslice, int ns, double* part,
+                              int batch, hipStream_t st) {
+  if (n < 1 || w < 1 || ldp < w || ldv < n || batch < 1 || batch > 65535 || ns < 1 || kslice < 16 || kslice % 16)
+    return hipErrorInvalidValue;
+  dg::Args a{};
+  a.M = a.N = w;
+  a.K = n;
+  a.alpha = 1.0;
+  a.A = a.B = V;
+  a.lda = a.ldb = ldv;
+  a.sa = a.sb = (long)w * ldv;
+  a.mode = dg::kSplit;
+  a.kslice = kslice;
+  a.C = part;
+  a.ldc = ldp;
+  a.zstride = (size_t)ldp * ldp;
+  a.sc = (long)ldp * ldp * ns;
+  return dg::launch<true, true, 64, 64, 16>(a, st, batch);
+}
+
 }  // namespace rnpx

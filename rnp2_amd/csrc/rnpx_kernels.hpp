@@ -275,13 +275,23 @@ template <typename T>
 hipError_t launch_tfactor(const T* gram, int ldg, int k, int nb, T* Tout, int ldt, hipStream_t st,
                           const unsigned* run_if = nullptr);
 
-// Gram of a clean V and tau into the layout launch_tfactor reads:
-// gram(j,c) = sum_r conj(V(r,j)) V(r,c) for j < c, tau_c on the diagonal.
-// Deterministic two-stage reduction over row chunks (scratch holds
-// nchunks * nb * nb elements).
+// The T factors of a stored factorization, all w-column blocks (w 32, 64 or
+// 128) of k reflectors at once.  launch_gram_blocks: gram[b] (w x w, blocks w*w
+// apart) in the layout launch_tfactor reads, from the clean V (n x k, zeros
+// above the unit diagonal) and tau; part holds gram_blocks_slices(n, k, w) *
+// ceil(k / w) * w * w elements, the slices added in order.  launch_tfactor_blocks:
+// T[b] (w x w) from gram[b]; at w = 128 its two 64-column diagonal parts (zero
+// elsewhere), to be joined by T12 = -T11 gram12 T22.
+int gram_blocks_slices(int n, int k, int w, int* kslice);
 template <typename T>
-hipError_t launch_gram(int n, int k, const T* V, long ldv, const T* tau, T* gram, int nb,
-                       T* scratch, int nchunks, hipStream_t st);
+hipError_t launch_gram_blocks(int n, int k, int w, const T* V, long ldv, const T* tau, T* gram, T* part,
+                              hipStream_t st);
+template <typename T>
+hipError_t launch_tfactor_blocks(const T* gram, int w, int k, T* Tout, hipStream_t st);
+hipError_t dgemm_gram_batched(int n, int w, int ldp, const double* V, long ldv, int kslice, int ns, double* part,
+                              int batch, hipStream_t st);
+hipError_t zgemm_gram_batched(int n, int w, int ldp, const zd* V, long ldv, int kslice, int ns, zd* part, int batch,
+                              hipStream_t st);
 
 // General matrix multiply on FP64 MFMA:
 //   C = alpha * op(A) * op(B) + beta * C,  op in {'N','T','C'}, column-major.

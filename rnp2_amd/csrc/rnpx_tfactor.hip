@@ -1,7 +1,8 @@
 // rnpx_tfactor.hip -- the T-factor kernel (the larft analogue,
 // Reflector::GenerateBlockTr "F","C", RNP/LA/Reflector.hpp:573-626) and the
-// Gram kernel that feeds it when V comes from a stored factorization
-// (QR::MultQ / QR::GenerateQ recompute T per block, QR.hpp:395, 557).
+// Grams that feed it when V comes from a stored factorization (QR::MultQ /
+// QR::GenerateQ recompute T per block, QR.hpp:395, 557; here every block's T
+// is formed before the first is applied, since all of V is there).
 //
 // RNP builds T column by column: T(0:c,c) = -tau_c T(0:c,0:c) V^H v_c.
 // Row j of that recurrence only touches row j of T, so here it runs as:
@@ -13,12 +14,26 @@
 // A tau_c == 0 column comes out zero, as at Reflector.hpp:584-587.
 #include "rnpx_kernels.hpp"
 
+#include <algorithm>
+
 namespace rnpx {
 
+// One workgroup per NB-column leaf of a set of w-column blocks (w a multiple of
+// NB; w = NB for a single T): leaf l belongs to block l NB / w, reads the
+// diagonal NB x NB part of that block's Gram (leading dimension ldg, blocks
+// gstride apart) and writes its w x NB strip of the block's T (zero outside the
+// diagonal part: the products that join two leaves fill in the part above).
+// kcols columns in all (a leaf beyond them: zeros).  Latency-bound (23 us, one leaf or fifty), so every
+// leaf of a stored factorization goes in one launch.
 template <typename T, int NB>
-__global__ __launch_bounds__(256) void tfactor_kernel(const T* __restrict__ gram, int ldg, int k,
-                                                       T* __restrict__ Tout, int ldt, const unsigned* run_if) {
+__global__ __launch_bounds__(256) void tfactor_kernel(const T* __restrict__ gram, int ldg, size_t gstride, int w,
+                                                       int kcols, T* __restrict__ Tout, int ldt, size_t tstride,
+                                                       const unsigned* run_if) {
   if (run_if && *run_if == 0u) return;
+  const int leaf0 = blockIdx.x * NB, blk = leaf0 / w, off = leaf0 - blk * w;
+  const int k = min(NB, kcols - leaf0);
+  gram += blk * gstride + (size_t)off * ldg + off;
+  Tout += blk * tstride + (size_t)off * ldt;
   constexpr int LEAF = 16;
   __shared__ T Gs[NB][NB + 1];  // Gs[l][c] = G(l,c), l < c; diagonal = tau
   __shared__ T Ts[NB][NB + 1];
@@ -73,9 +88,9 @@ __global__ __launch_bounds__(256) void tfactor_kernel(const T* __restrict__ gram
     }
     __syncthreads();
   }
-  for (int e = tid; e < NB * NB; e += 256) {
-    const int l = e % NB, c = e / NB;
-    Tout[(size_t)l + (size_t)c * ldt] = Ts[l][c];
+  for (int e = tid; e < w * NB; e += 256) {
+    const int l = e % w, c = e / w, d = l - off;
+    Tout[(size_t)l + (size_t)c * ldt] = (d >= 0 && d < NB) ? Ts[d][c] : S<T>::zero();
   }
 }
 
@@ -84,71 +99,85 @@ hipError_t launch_tfactor(const T* gram, int ldg, int k, int nb, T* Tout, int ld
                           const unsigned* run_if) {
   if (k < 0 || k > nb || ldg < nb || ldt < nb) return hipErrorInvalidValue;
   if (nb == 16)
-    hipLaunchKernelGGL((tfactor_kernel<T, 16>), dim3(1), dim3(256), 0, st, gram, ldg, k, Tout, ldt, run_if);
+    hipLaunchKernelGGL((tfactor_kernel<T, 16>), dim3(1), dim3(256), 0, st, gram, ldg, (size_t)0, nb, k, Tout, ldt,
+                       (size_t)0, run_if);
   else if (nb == 32)
-    hipLaunchKernelGGL((tfactor_kernel<T, 32>), dim3(1), dim3(256), 0, st, gram, ldg, k, Tout, ldt, run_if);
+    hipLaunchKernelGGL((tfactor_kernel<T, 32>), dim3(1), dim3(256), 0, st, gram, ldg, (size_t)0, nb, k, Tout, ldt,
+                       (size_t)0, run_if);
   else if (nb == 64)
-    hipLaunchKernelGGL((tfactor_kernel<T, 64>), dim3(1), dim3(256), 0, st, gram, ldg, k, Tout, ldt, run_if);
+    hipLaunchKernelGGL((tfactor_kernel<T, 64>), dim3(1), dim3(256), 0, st, gram, ldg, (size_t)0, nb, k, Tout, ldt,
+                       (size_t)0, run_if);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
-// Gram stage 1: chunk s of the rows, one workgroup per (chunk, column c):
-// part[s](j,c) = sum_{r in chunk} conj(V(r,j)) V(r,c) for j <= c.
 template <typename T>
-__global__ __launch_bounds__(256) void gram_partial_kernel(int n, int k, const T* __restrict__ V, long ldv,
-                                                           int rows_per_chunk, int nb, T* __restrict__ part) {
-  const int s = blockIdx.x, c = blockIdx.y;
-  const int r0 = s * rows_per_chunk, r1 = min(n, r0 + rows_per_chunk);
-  __shared__ T red[4][64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  T* out = part + (size_t)s * nb * nb + (size_t)c * nb;
-  for (int j0 = 0; j0 <= c; j0 += 64) {
-    // each wave takes every 4th row; lanes own column j0 + lane
-    const int j = j0 + lane;
-    T acc = S<T>::zero();
-    if (j <= c) {
-      for (int r = r0 + wave; r < r1; r += 4)
-        acc = acc + S<T>::cmul(V[(size_t)r + (size_t)j * ldv], V[(size_t)r + (size_t)c * ldv]);
-    }
-    red[wave][lane] = acc;
-    __syncthreads();
-    if (wave == 0 && j <= c) out[j] = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
-    __syncthreads();
-  }
-}
-
-template <typename T>
-__global__ void gram_final_kernel(int k, int nb, int nchunks, const T* __restrict__ part,
-                                  const T* __restrict__ tau, T* __restrict__ gram) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= nb * nb) return;
-  const int j = e % nb, c = e / nb;
-  T s = S<T>::zero();
-  if (c < k && j < c) {
-    s = sum_strided(part + (size_t)c * nb + j, nchunks, (size_t)nb * nb);
-  } else if (c < k && j == c) {
-    s = tau[c];
-  }
-  gram[(size_t)j + (size_t)c * nb] = s;
-}
-
-template <typename T>
-hipError_t launch_gram(int n, int k, const T* V, long ldv, const T* tau, T* gram, int nb,
-                       T* scratch, int nchunks, hipStream_t st) {
-  if (k < 1 || k > nb || n < k || nchunks < 1) return hipErrorInvalidValue;
-  const int rpc = (n + nchunks - 1) / nchunks;
-  hipLaunchKernelGGL((gram_partial_kernel<T>), dim3(nchunks, k), dim3(256), 0, st, n, k, V, ldv, rpc, nb, scratch);
-  hipLaunchKernelGGL((gram_final_kernel<T>), dim3((nb * nb + 255) / 256), dim3(256), 0, st, k, nb, nchunks,
-                     scratch, tau, gram);
+hipError_t launch_tfactor_blocks(const T* gram, int w, int k, T* Tout, hipStream_t st) {
+  if (k < 1) return hipErrorInvalidValue;
+  const size_t ws = (size_t)w * w;
+  if (w == 32)
+    hipLaunchKernelGGL((tfactor_kernel<T, 32>), dim3((k + 31) / 32), dim3(256), 0, st, gram, w, ws, w, k, Tout, w, ws,
+                       (const unsigned*)nullptr);
+  else if (w == 64 || w == 128)
+    hipLaunchKernelGGL((tfactor_kernel<T, 64>), dim3((k + w - 1) / w * (w / 64)), dim3(256), 0, st, gram, w, ws, w, k, Tout, w, ws,
+                       (const unsigned*)nullptr);
+  else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
-template hipError_t launch_tfactor<double>(const double*, int, int, int, double*, int, hipStream_t,
-                                           const unsigned*);
-template hipError_t launch_tfactor<zd>(const zd*, int, int, int, zd*, int, hipStream_t, const unsigned*);
-template hipError_t launch_gram<double>(int, int, const double*, long, const double*, double*, int, double*, int,
-                                        hipStream_t);
-template hipError_t launch_gram<zd>(int, int, const zd*, long, const zd*, zd*, int, zd*, int, hipStream_t);
+// gram[b](j, c), j < c, of every block from its ns row slices (added in slice
+// order), tau on the diagonal, zero below it and beyond the k columns.
+template <typename T>
+__global__ void gram_sum_blocks_kernel(int k, int w, int ns, const T* __restrict__ part, const T* __restrict__ tau,
+                                       T* __restrict__ gram) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.y;
+  if (e >= w * w) return;
+  const size_t ws = (size_t)w * w;
+  const int j = e % w, c = e / w, col = b * w + c;
+  T s = S<T>::zero();
+  if (col < k && j < c)
+    s = sum_strided(part + (size_t)b * ns * ws + e, ns, ws);
+  else if (col < k && j == c)
+    s = tau[col];
+  gram[b * ws + e] = s;
+}
+
+int gram_blocks_slices(int n, int k, int w, int* kslice) {
+  const int nblk = (k + w - 1) / w, tiles = (w <= 64 ? 1 : 4) * nblk;
+  // about three workgroups per CU in all, slices of at least 256 rows
+  int ns = std::max(1, std::min({64, n / 256, 768 / tiles}));
+  *kslice = ((n + ns - 1) / ns + 15) / 16 * 16;
+  return (n + *kslice - 1) / *kslice;
+}
+
+template <typename T>
+hipError_t launch_gram_blocks(int n, int k, int w, const T* V, long ldv, const T* tau, T* gram, T* part,
+                              hipStream_t st) {
+  if (k < 1 || n < k || ldv < n) return hipErrorInvalidValue;
+  int kslice = 0;
+  const int ns = gram_blocks_slices(n, k, w, &kslice), full = k / w, rest = k - full * w;
+  const size_t ws = (size_t)w * w;
+  for (int r = 0; r < 2; ++r) {  // the full blocks, then a narrower last one
+    const int nb = r == 0 ? full : (rest > 0), cols = r == 0 ? w : rest;
+    if (nb == 0) continue;
+    const T* Vr = V + (r == 0 ? 0 : (size_t)full * w * ldv);
+    T* pr = part + (r == 0 ? 0 : full * ns * ws);
+    if constexpr (S<T>::cplx)
+      RNPX_LAUNCH_CHECK(zgemm_gram_batched(n, cols, w, Vr, ldv, kslice, ns, pr, nb, st));
+    else
+      RNPX_LAUNCH_CHECK(dgemm_gram_batched(n, cols, w, Vr, ldv, kslice, ns, pr, nb, st));
+  }
+  hipLaunchKernelGGL((gram_sum_blocks_kernel<T>), dim3((unsigned)((ws + 255) / 256), full + (rest > 0)), dim3(256), 0,
+                     st, k, w, ns, part, tau, gram);
+  return hipGetLastError();
+}
+
+#define RNPX_TF_INST(T)                                                                                       \
+  template hipError_t launch_tfactor<T>(const T*, int, int, int, T*, int, hipStream_t, const unsigned*);      \
+  template hipError_t launch_tfactor_blocks<T>(const T*, int, int, T*, hipStream_t);                          \
+  template hipError_t launch_gram_blocks<T>(int, int, int, const T*, long, const T*, T*, T*, hipStream_t);
+RNPX_TF_INST(double)
+RNPX_TF_INST(zd)
+#undef RNPX_TF_INST
 
 }  // namespace rnpx

@@ -103,6 +103,7 @@ struct Args {
   int kslice;
   int tilesM, tilesN;
   int conja;  // op(A) = 'C'
+  long sa, sb, sc;  // strided batch (grid y): elements between the problems' A, B, C
 };
 
 // Workgroup -> (tile m, tile n, split z): contiguous chunks per XCD, then
@@ -124,12 +125,16 @@ __device__ inline void tile_of(const Args& a, int w, int nwg, int& tm, int& tn, 
 }
 
 template <int MODE, bool AKC, int BM, int BN, int BK>
-__global__ __launch_bounds__(kThreads) void zgemm_kernel(Args a) {
+__global__ __launch_bounds__(kThreads) void zgemm_kernel(Args a0) {
   using OA = ZOp<AKC, BM, BK>;
   using OB = ZOp<true, BN, BK>;  // op(B) = N: contiguous along K
   constexpr int FM = BM / 32, FN = BN / 32;
   __shared__ double Ar[2][OA::ELEMS], Ai[2][OA::ELEMS];
   __shared__ double Br[2][OB::ELEMS], Bi[2][OB::ELEMS];
+  Args a = a0;  // problem blockIdx.y of a strided batch (0 for one product)
+  a.A += (size_t)blockIdx.y * a0.sa;
+  a.B += (size_t)blockIdx.y * a0.sb;
+  a.C += (size_t)blockIdx.y * a0.sc;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
@@ -237,10 +242,10 @@ __global__ __launch_bounds__(kThreads) void zgemm_kernel(Args a) {
 }
 
 template <bool AKC, int BM, int BN, int BK>
-static hipError_t launch(Args a, int ns, hipStream_t st) {
+static hipError_t launch(Args a, int ns, hipStream_t st, int batch = 1) {
   a.tilesM = (a.M + BM - 1) / BM;
   a.tilesN = (a.N + BN - 1) / BN;
-  const dim3 grid((unsigned)(a.tilesM * a.tilesN * ns)), block(kThreads);
+  const dim3 grid((unsigned)(a.tilesM * a.tilesN * ns), (unsigned)batch), block(kThreads);
   switch (a.mode) {
     case kCInit: hipLaunchKernelGGL((zgemm_kernel<kCInit, AKC, BM, BN, BK>), grid, block, 0, st, a); break;
     case kSplit: hipLaunchKernelGGL((zgemm_kernel<kSplit, AKC, BM, BN, BK>), grid, block, 0, st, a); break;
@@ -299,6 +304,28 @@ hipError_t zgemm_mfma(char ta, char tb, int M, int N, int K, zd alpha, const zd*
   }
   if (M <= 32) return zg::launch<false, 32, 64, BK>(a, ns, st);
   return zg::launch<false, 64, 64, BK>(a, ns, st);
+}
+
+// Batched Grams V_b^H V_b, as dgemm_gram_batched.
+hipError_t zgemm_gram_batched(int n, int w, int ldp, const zd* V, long ldv, int kslice, int ns, zd* part, int batch,
+                              hipStream_t st) {
+  if (n < 1 || w < 1 || ldp < w || ldv < n || batch < 1 || batch > 65535 || ns < 1 || kslice < 16 || kslice % 16)
+    return hipErrorInvalidValue;
+  zg::Args a{};
+  a.M = a.N = w;
+  a.K = n;
+  a.alpha = S<zd>::one();
+  a.A = a.B = V;
+  a.lda = a.ldb = ldv;
+  a.sa = a.sb = (long)w * ldv;
+  a.conja = 1;
+  a.mode = zg::kSplit;
+  a.kslice = kslice;
+  a.C = part;
+  a.ldc = ldp;
+  a.zstride = (size_t)ldp * ldp;
+  a.sc = (long)ldp * ldp * ns;
+  return zg::launch<true, 64, 64, 16>(a, ns, st, batch);
 }
 
 }  // namespace rnpx
