@@ -71,6 +71,8 @@ struct Handle {
   Buffer lqbuf;                            // A^H for the LQ routines
   Buffer qlbuf;                            // reversed reflectors and tau (QL, RQ)
   Buffer lubuf;                            // LU panel scratch, Solve's permutation and gather
+  Buffer lull;                             // real LU panels' tagged hand-off words
+  unsigned lu_tag = 0;                     // the last tag used in them (0: words not cleared yet)
   Buffer rfbuf;                            // RefineSolution's residual and |op(A)||x| + |b|
   Buffer invbuf;                           // LU::Invert's n x n right-hand side and U's diagonal
   Buffer exbuf;                            // non-finite flag, trim limits, T and work of the exact path
@@ -84,7 +86,7 @@ struct Handle {
   std::vector<Buffer*> buffers() {
     return {&vbuf, &vfull, &gram, &tbuf, &wbuf, &zbuf, &part, &ppart, &rowbuf, &sync, &flag, &misc,
             &vbuf2, &gram2, &tbuf2, &stage1, &stage2, &stage3, &lsbuf, &lsnrm, &cqr_part, &cqr_gsum,
-            &cqr_scratch, &wbuf2, &zbuf2, &part2, &misc2, &trsm_flags, &lqbuf, &qlbuf, &lubuf, &rfbuf, &invbuf, &exbuf, &exsave, &rinv, &zcqr, &gemvbuf};
+            &cqr_scratch, &wbuf2, &zbuf2, &part2, &misc2, &trsm_flags, &lqbuf, &qlbuf, &lubuf, &lull, &rfbuf, &invbuf, &exbuf, &exsave, &rinv, &zcqr, &gemvbuf};
   }
   hipError_t sync_all_streams();       // the handle's stream, panel stream and partition streams
   void* batch = nullptr;               // batched-call descriptor buffers

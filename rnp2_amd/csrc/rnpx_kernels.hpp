@@ -146,6 +146,12 @@ struct LuPanelArgs {
   void* A; long lda;    // panel top-left (T = double or zd)
   int* piv;             // out: jb pivot rows, relative to the panel top
   int* zero_last;       // out: the last column with an exact zero pivot, -1 if none
+  int* moves;           // out: count (zero at launch), then (from, to) rows that moved: kLuMoveWords
+  // real panels: 2 * 128 slots of kLuSlotWords hand-off words, and the tag of
+  // the panel's first column (tag0 .. tag0 + 63 were never used in them before)
+  unsigned long long* ll;
+  unsigned tag0;
+  // complex panels
   double* part;         // scratch: 2 * G * (2 + 2*64) doubles (candidates)
   double* rowc;         // scratch: 2 * 2*64 doubles (row c)
   unsigned* sync;       // 2 words per column (an arrival counter used), zero at launch
@@ -154,18 +160,24 @@ struct LuPanelArgs {
 #define RNPX_LU_GLOBAL(a)                                                                              \
   do {                                                                                                 \
     (a).A = as_global((a).A); (a).piv = as_global((a).piv); (a).zero_last = as_global((a).zero_last); \
+    (a).moves = as_global((a).moves); (a).ll = as_global((a).ll);                                      \
     (a).part = as_global((a).part); (a).rowc = as_global((a).rowc);                                    \
     (a).sync = as_global((a).sync); (a).abortf = as_global((a).abortf);                               \
   } while (0)
 constexpr int kLuPanelNB = 64;
 constexpr int kLuPartPerGroup = 2 + 2 * kLuPanelNB;
-// Rows per workgroup for an mp-row panel within max_groups workgroups (64,
-// 128 or 256; 0 when the panel is too tall).
+constexpr int kLuMaxMoves = 2 * kLuPanelNB;          // the panel's first 64 rows and 64 pivot rows
+constexpr int kLuMoveWords = 1 + 2 * kLuMaxMoves;
+constexpr int kLuRowThreads = 512;                   // real panels: rows per workgroup
+constexpr int kLuSlotWords = 2 * kLuPanelNB + 8;     // a row in halves, then the candidate
+// Rows per workgroup for an mp-row panel within max_groups workgroups (real
+// 512, complex 64 or 128; 0 when the panel is too tall).
 int lu_panel_rows(int mp, int max_groups, int cplx);
 template <typename T>
 hipError_t launch_lu_panel(const LuPanelArgs& a, int rw, hipStream_t st);
+// moves: the panel's list, relative to row j.
 template <typename T>
-hipError_t launch_lu_laswp(int j, int jb, const int* piv, T* A, long lda, int c0, int ncols, hipStream_t st);
+hipError_t launch_lu_laswp(int j, const int* moves, T* A, long lda, int c0, int ncols, hipStream_t st);
 template <typename T>
 hipError_t launch_lu_trsm(int jb, const T* L, long ldl, T* B, long ldb, int ncols, hipStream_t st);
 template <typename T>

@@ -1,8 +1,7 @@
 // rnpx_lu_driver.cpp -- LU::Factor and LU::Solve (RNP/LA/LU.hpp:77-144) on the
 // device: the blocked loop of LU::Factor with each 64-column panel factored
 // by one cooperative launch, the panel's row interchanges applied to the
-// other columns, U12 by substitution and the trailing update as a GEMM
-// (rocBLAS DGEMM for real matrices, the library's MFMA GEMM otherwise).
+// other columns, U12 by substitution and the trailing update as an MFMA GEMM.
 //
 // Return value: the reference's arithmetic (LU.hpp:63-74, 94-96, 112-113):
 // a panel whose last exact-zero pivot is its column z > 0 reports
@@ -32,16 +31,27 @@ int getrf_dev(Handle* h, int m, int n, T* A, long lda, int* piv_host, int* info)
   const int maxg = std::min(256, h->num_cus);
   const int rw = lu_panel_rows(m, maxg, S<T>::cplx ? 1 : 0);
   if (rw == 0) return RNPX_ERR_UNSUPPORTED;
-  // scratch: candidates, row c, results (doubles); sync words; zero-pivot
-  // columns and relative pivots (ints)
-  const size_t nd = (size_t)2 * 256 * kLuPartPerGroup + 4 * nb + 2 * nb;
-  const size_t bytes = sizeof(double) * nd + sizeof(unsigned) * 2 * nb + sizeof(int) * ((size_t)npan + k);
-  RNPX_TRY(h->lubuf.ensure(bytes, h));
+  // scratch: per panel the zero-pivot column, the relative pivots and the
+  // moved rows (ints); complex panels' candidates, row c and sync words
+  const size_t nd = S<T>::cplx ? (size_t)2 * 256 * kLuPartPerGroup + 4 * nb + 2 * nb : 0;
+  const size_t nints = (size_t)npan + k + (size_t)npan * kLuMoveWords;
+  RNPX_TRY(h->lubuf.ensure(sizeof(double) * nd + sizeof(unsigned) * 2 * nb + sizeof(int) * nints, h));
   double* part = (double*)h->lubuf.p;
   double* rowc = part + (size_t)2 * 256 * kLuPartPerGroup;
-  unsigned* sync = (unsigned*)(rowc + 6 * nb);
+  unsigned* sync = (unsigned*)(part + nd);
   int* zl = (int*)(sync + 2 * nb);
   int* prel = zl + npan;
+  int* moves = prel + k;
+  RNPX_TRY(launch_zero_u32((unsigned*)moves, npan * kLuMoveWords, h->stream));
+  if (!S<T>::cplx) {
+    // tags only grow; the words are cleared when new or when the tags run out
+    const size_t words = (size_t)2 * 128 * kLuSlotWords, before = h->lull.bytes;
+    RNPX_TRY(h->lull.ensure(sizeof(unsigned long long) * words, h));
+    if (h->lull.bytes != before || h->lu_tag > 0xFFFFFFFFu - (unsigned)(npan + 1) * nb) {
+      RNPX_TRY(launch_zero_u32((unsigned*)h->lull.p, (int)(2 * words), h->stream));
+      h->lu_tag = 0;
+    }
+  }
   // Panel pi factors columns [j, j+jb).  Its update of the columns to the
   // right is split: the next panel's columns are brought up to date on the
   // panel stream right behind it (so the chain of panels crosses no stream),
@@ -60,14 +70,18 @@ int getrf_dev(Handle* h, int m, int n, T* A, long lda, int* piv_host, int* info)
   }
   auto panel = [&](int pi) -> int {
     const int j = pi * nb, jb = std::min(nb, k - j), mp = m - j;
-    RNPX_TRY(launch_zero_u32(sync, 2 * nb, ps));
-    LuPanelArgs pa;
+    if (S<T>::cplx) RNPX_TRY(launch_zero_u32(sync, 2 * nb, ps));
+    LuPanelArgs pa{};
     pa.mp = mp;
     pa.jb = jb;
     pa.A = A + (size_t)j + (size_t)j * lda;
     pa.lda = lda;
     pa.piv = prel + j;
     pa.zero_last = zl + pi;
+    pa.moves = moves + (size_t)pi * kLuMoveWords;
+    pa.ll = (unsigned long long*)h->lull.p;
+    pa.tag0 = h->lu_tag + 1;
+    h->lu_tag += nb;
     pa.part = part;
     pa.rowc = rowc;
     pa.sync = sync;
@@ -80,7 +94,7 @@ int getrf_dev(Handle* h, int m, int n, T* A, long lda, int* piv_host, int* info)
   auto right = [&](int pi, int c0, int nc, hipStream_t s) -> int {
     if (nc <= 0) return RNPX_OK;
     const int j = pi * nb, jb = std::min(nb, k - j);
-    RNPX_TRY(launch_lu_laswp<T>(j, jb, prel + j, A, lda, c0, nc, s));
+    RNPX_TRY(launch_lu_laswp<T>(j, moves + (size_t)pi * kLuMoveWords, A, lda, c0, nc, s));
     RNPX_TRY(launch_lu_trsm<T>(jb, A + (size_t)j + (size_t)j * lda, lda, A + (size_t)j + (size_t)c0 * lda, lda, nc, s));
     if (j + jb < m) {
       T* L21 = A + (size_t)(j + jb) + (size_t)j * lda;
@@ -105,7 +119,7 @@ int getrf_dev(Handle* h, int m, int n, T* A, long lda, int* piv_host, int* info)
       if ((e = panel(pi + 1))) return e;
       cr = c1 + jb2;
     }
-    if (j > 0) RNPX_TRY(launch_lu_laswp<T>(j, jb, prel + j, A, lda, 0, j, st));
+    if (j > 0) RNPX_TRY(launch_lu_laswp<T>(j, moves + (size_t)pi * kLuMoveWords, A, lda, 0, j, st));
     if ((e = right(pi, cr, n - cr, st))) return e;
     if (look) RNPX_TRY(hipEventRecord(h->ev_rest, st));
   }
