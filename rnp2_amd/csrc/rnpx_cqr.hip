@@ -49,6 +49,7 @@
 #include "rnpx_small64.hpp"
 #include "rnpx_team.hpp"
 
+#include <algorithm>
 #include <cstdlib>
 
 namespace rnpx {
@@ -193,13 +194,15 @@ __device__ __forceinline__ void times_upper(double (*Ab)[LDA_S], const double (*
   for (int q = 0; q < RT; ++q) {
     const int t = wave + 4 * q;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      acc[q][c] = f64x4{0.0, 0.0, 0.0, 0.0};
-      for (int k0 = 0; k0 < 16 * (c + 1); k0 += 4) {  // X[k][16c..] = 0 for k >= 16(c+1)
-        const double x = Ab[16 * t + (lane & 15)][k0 + (lane >> 4)];
-        const double y = X[k0 + (lane >> 4)][16 * c + (lane & 15)];
-        acc[q][c] = mfma16(x, y, acc[q][c]);
-      }
+    for (int c = 0; c < 4; ++c) acc[q][c] = f64x4{0.0, 0.0, 0.0, 0.0};
+    // the reduction outside, a step's four columns' MFMAs independent of one
+    // another
+#pragma unroll
+    for (int k0 = 0; k0 < 64; k0 += 4) {
+      const double x = Ab[16 * t + (lane & 15)][k0 + (lane >> 4)];
+#pragma unroll
+      for (int c = k0 / 16; c < 4; ++c)  // X[k][16c..] = 0 for k >= 16(c+1)
+        acc[q][c] = mfma16(x, X[k0 + (lane >> 4)][16 * c + (lane & 15)], acc[q][c]);
     }
   }
   __syncthreads();
@@ -223,16 +226,19 @@ __device__ __forceinline__ void upper_product_row(const double (*A)[LDA_S], cons
                                   f64x4 (&acc)[4], int lane, int wave) {
   const int ti = wave;
 #pragma unroll
-  for (int tj = 0; tj < 4; ++tj) {
-    acc[tj] = f64x4{0.0, 0.0, 0.0, 0.0};
-    if (tj < ti) continue;
-    for (int k0 = 16 * ti; k0 < 16 * (tj + 1); k0 += 4) {
+  for (int tj = 0; tj < 4; ++tj) acc[tj] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) {
+    // (A's blocks left of its diagonal count as zero)
+#pragma unroll
+    for (int k0 = 16 * kb; k0 < 16 * kb + 16; k0 += 4) {
       const int i = 16 * ti + (lane & 15), k = k0 + (lane >> 4);
       double x = A[i][k];
-      if (mask_a && k < i) x = 0.0;
+      if (kb < ti || (mask_a && k < i)) x = 0.0;
       if (dcol) x *= dcol[k];
-      const double y = TB ? B[16 * tj + (lane & 15)][k] : B[k][16 * tj + (lane & 15)];
-      acc[tj] = mfma16(x, y, acc[tj]);
+#pragma unroll
+      for (int tj = kb; tj < 4; ++tj)
+        acc[tj] = mfma16(x, TB ? B[16 * tj + (lane & 15)][k] : B[k][16 * tj + (lane & 15)], acc[tj]);
     }
   }
 }
@@ -347,6 +353,7 @@ __global__ __launch_bounds__(256) void cqr_panel_kernel(CqrArgs a) {
   gram_allreduce(a, 0, G, g, tid, &slot);
   load_gram(a.gsum, M1, tid);
   __syncthreads();
+  if (tid < NB) gdiag[tid] = M1[tid][tid];
   const bool ok1 = small64::chol64<LDA_S>(&M1[0][0], &M2[0][0], tmpb, gdiag, &okf, tid);  // M1 = R1, M2 = R1^-1
   if (!ok1) {
     // Every workgroup factored the same Gram and takes this branch; nothing
@@ -378,6 +385,7 @@ __global__ __launch_bounds__(256) void cqr_panel_kernel(CqrArgs a) {
     }
     __syncthreads();
   } else {
+    if (tid < NB) gdiag[tid] = M1[tid][tid];
     small64::chol64<LDA_S>(&M1[0][0], &M2[0][0], tmpb, gdiag, &okf, tid);
   }
   times_upper<RW>(Ab, M2, lane, wave);
@@ -387,7 +395,7 @@ __global__ __launch_bounds__(256) void cqr_panel_kernel(CqrArgs a) {
     // LU of Q_top - D, published with U^-1.
     for (int e = tid; e < NB * NB; e += 256) M1[e / NB][e % NB] = Ab[e / NB][e % NB];
     __syncthreads();
-    small64::lu64<LDA_S>(&M1[0][0], rowbuf, &M2[0][0], tmpb, tid);  // M1 = U and L, M2 = U^-1
+    small64::lu64<LDA_S>(&M1[0][0], rowbuf, &M2[0][0], tmpb, &okf, tid);  // M1 = U and L, M2 = U^-1
     for (int e = tid; e < NB * NB; e += 256) {
       ulp[e] = M1[e / NB][e % NB];
       uinv[e] = M2[e / NB][e % NB];
@@ -474,134 +482,261 @@ __global__ __launch_bounds__(256) void cqr_panel_kernel(CqrArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// One outer block of 128 columns in one launch: panel 1 (columns 0..63) by
-// CholeskyQR2 + reconstruction as above, its block reflector applied to
-// panel 2's columns (W = V1^T A2 by a grid reduction, Z = T1^T W,
-// A2 -= V1 Z, all in LDS), panel 2 (rows 64.., columns 64..127) the same
-// way over workgroups 1.., and the merged compact-WY form
-//   V = [V1 | (0; V2)],  T = [T1, -T1 (V1^T V2) T2; 0, T2]
-// with V1^T V2 by a third grid reduction.  This replaces, per outer block,
-// two panel launches and the six small products around them.  Workgroup g
-// holds rows [64 g, 64 g + 64) of both panels in LDS for the whole launch;
-// nothing is written to A before panel 2 has passed its tests, so a
-// rejection of either panel leaves A untouched and workgroup 0 refactors
-// all 128 columns column by column instead.  Each panel's T is formed by the
-// workgroup that factored its LU (still in LDS) while the next grid
-// reduction completes: T1 by workgroup 0, T2 and the merge by workgroup 1.
+// One outer block of up to 128 columns in one launch, by CholeskyQR2 of all
+// its columns at once and Householder reconstruction in two 64-column halves
+// (one when w <= 64).  Workgroup g holds rows [64 g, 64 g + 64) of both halves
+// in LDS; columns beyond w and rows beyond mp are zero (their Gram diagonal is
+// taken as one), so any width and height of a factorization's end runs here.
+//   1. The Gram of the block [A1 A2] by one grid reduction; every workgroup
+//      factors it itself: R11 = chol(G11), R12 = R11^-T G12,
+//      R22 = chol(G22 - R12^T R12); Q1 = A1 R11^-1, Q2 = (A2 - Q1 R12) R22^-1.
+//   2. The Gram I + E of [Q1 Q2] by a second reduction.  |E| <= 2^-40: first
+//      order, R = I + triu(E) - diag(E)/2 (exact to |E|^2).  |E| <= 2^-27:
+//      factored as in 1, which leaves Q orthonormal to working precision.
+//      |E| <= 2^-3: factored, and the Gram taken again (a block of condition
+//      up to about 1e7; CholeskyQR iterated).  Otherwise the block is
+//      rejected, as it is when a pivot falls below 2^-40 of its column's
+//      squared norm, a squared norm is outside [2^-600, 2^600] or a value is
+//      not finite.  Every workgroup takes the same decision from the same
+//      reduced Gram, and A is untouched until the block is accepted; a rejected
+//      block is refactored column by column by workgroup 0.
+//   3. Reconstruction [Q1 Q2] - [D; 0] = L U without another reduction:
+//      workgroup 0 factors Q1's top block (L11, U11, D1) and forms
+//      U12 = L11^-1 Q2(0:64), everybody V1 = Q1 U11^-1 and Q2 - V1 U12,
+//      workgroup 1 factors that one's rows 64..127 (L22, U22, D2), everybody
+//      V2 = (Q2 - V1 U12) U22^-1.  tau_j = -U_jj D_j,
+//      T = -U D L^-T: T11 = -U11 D1 L11^-T, T22 = -U22 D2 L22^-T and
+//      T12 = -(T11 L21^T + U12 D2) L22^-T with L21 = V1(64:128).
+//      R = D times the product of the passes' factors, by workgroup 2 beside
+//      the two LUs.
+// In a square last block (mp == w) the last column has no entries below it and
+// so no reflector (tau = 0, Reflector.hpp:122-125): there D takes the running
+// pivot's own sign and T's column is zero.  Any other column whose entries
+// below the diagonal are exactly zero has no reflector either, which the
+// reconstruction cannot tell from tiny entries (both give tau = 2 to rounding):
+// with zero_tails such a block (a running pivot within 2^-40 of one) is rejected.
+// Bound by the chain of two grid reductions, two Cholesky and two LU
+// factorizations of 64 x 64.  Against two 64-column panels joined inside the
+// launch (six reductions, the second panel's Gram after the first one's
+// reconstruction; 370 KB of unrolled code where this is 96 KB, most of it cold in
+// the instruction cache): 201 -> 168 us per block at 1931 rows and below; the
+// factorization of 1931 x 1207, whose last 55 columns also run here now,
+// 2.70 -> 2.24 ms, 8192^2 29.4 -> 27.1 ms, 250 x 64 0.11 ms as before,
+// 100 x 64 0.32 -> 0.11 ms, 100 x 100 0.55 -> 0.27 ms.
 // ---------------------------------------------------------------------------
 namespace {
 
-constexpr int kBlkPassWords = 32;                 // per reduction pass
-constexpr int kBlkPub1 = 6 * kBlkPassWords;        // panel 1's LU published
-constexpr int kBlkPubT1 = kBlkPub1 + 1;            // T1 published
-constexpr int kBlkPub2 = kBlkPub1 + 2;             // panel 2's LU published
-constexpr int kBlkResident = kBlkPub1 + 3;         // workgroups started (for the gate below)
-static_assert(kBlkPub2 < kCqrBlockSyncWords, "block sync words");
-constexpr int kCross = 16 * 256;                   // 64x64 product partial (16 tiles)
-// scratch (doubles)
-constexpr int kBR1a = 0, kBU1i = 4096, kBD1 = 12288, kBTau1 = 12352, kBRF1 = 12416, kBT1 = 16512,
-              kBR1b = 20608, kBU2i = 24704, kBD2 = 32896, kBG = 32960, kBTF = 49344;
-static_assert(kBTF + 16384 <= kCqrBlockScratch, "block scratch");
+constexpr int kBlkPassWords = 32;                 // per reduction pass (at most four)
+constexpr int kBlkPub1 = 6 * kBlkPassWords;        // LU of the first half published
+constexpr int kBlkPubU12 = kBlkPub1 + 1;           // U12 published
+constexpr int kBlkPubT1 = kBlkPub1 + 2;            // T11 published
+constexpr int kBlkPub2 = kBlkPub1 + 3;             // LU of the second half published
+constexpr int kBlkResident = kBlkPub1 + 4;         // workgroups started (for the gate below)
+static_assert(kBlkResident < kCqrBlockSyncWords, "block sync words");
+constexpr int kCross = 16 * 256;                   // a 64x64 product in 16 tiles
+constexpr int kBlkElems = kCqrBlockPart;           // upper tiles of a 128x128 Gram: G11, G12, G22
+static_assert(2 * kGramElems + kCross == kBlkElems, "Gram layout: tiles 0..9, 10..25, 26..35");
+constexpr int kBlkPasses = 3;                      // Cholesky passes at most (and one first-order pass)
+constexpr double kThirdPass = 0x1p-3;
+constexpr unsigned kRejected = 2u;                 // flag value: the block goes column by column
+// scratch (doubles): R11, R12, R22 of each pass, then the published blocks;
+// the column-wise refactorization's Gram and T reuse the front
+constexpr int kBR = 0, kBU1i = 3 * 4096 * (kBlkPasses + 1), kBU12 = kBU1i + 4096, kBT1 = kBU12 + 4096,
+              kBU2i = kBT1 + 4096, kBD1 = kBU2i + 4096, kBD2 = kBD1 + 64, kBG = 0, kBTF = 16384;
+static_assert(kBD2 + 64 <= kCqrBlockScratch && kBTF + 16384 <= kCqrBlockScratch, "block scratch");
 
-// Reduction of Gp partials (ELEMS doubles each, kCross apart from a.part)
-// into gs, by reduce-scatter.  Contributors arrive on the pass's first
-// counter once their partial is stored.  Each helper workgroup (index hi of
-// Hn; hi < 0 for none) then waits for all Gp arrivals, sums its slice of
-// the entries over the partials in a fixed order (so the result does not
-// depend on timing), stores it and arrives on the second counter; the sum
-// is complete once Hn helpers have arrived (blk_wait).  red: 256 doubles of
-// LDS scratch.
-template <int ELEMS>
-__device__ __forceinline__ void blk_contribute(const CqrBlockArgs& a, int pass, bool contrib, int Gp, int hi, int Hn,
-                                               double* gs, double* red, int tid, unsigned* slot) {
+// wait_flag, and the flag's value in every thread.
+__device__ __forceinline__ unsigned wait_verdict(unsigned* flag, unsigned* abortf, unsigned* slot) {
+  wait_flag(flag, abortf);
+  if (threadIdx.x == 0) *slot = __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  const unsigned v = *slot;
+  __syncthreads();
+  return v;
+}
+
+// Reduction of G partials (elems doubles each, kBlkElems apart from a.part)
+// into gs, by reduce-scatter.  Every workgroup arrives on the pass's first
+// counter once its partial is stored, waits for all arrivals, sums its slice
+// of the entries over the partials in a fixed order (so the result does not
+// depend on timing), stores it and arrives on the second counter; the sum is
+// complete once all have arrived there.  red: 512 doubles of LDS scratch.
+__device__ __forceinline__ void blk_allreduce(const CqrBlockArgs& a, int elems, int pass, int g, int G, double* gs,
+                                              double* red, int tid, unsigned* slot) {
   unsigned* sw = a.sync + pass * kBlkPassWords;
-  if (contrib) arrive(&sw[0], slot);
-  if (hi < 0) return;
-  wait_count(&sw[0], (unsigned)Gp, a.abortf);
-  const int S = (ELEMS + Hn - 1) / Hn;  // slice length
-  const int e0 = hi * S, len = min(S, ELEMS - e0);
-  if (S <= 128) {
-    // P threads per entry, each over every P-th partial; then the P sums
-    const int P = 256 / S, j = tid / S, x = tid % S;
-    double sum = 0.0;
-    if (j < P && x < len) {
-      const double* src = a.part + e0 + x;
-#pragma unroll 8
-      for (int q = j; q < Gp; q += P) sum += src[(size_t)q * kCross];
+  arrive(&sw[0], slot);
+  wait_count(&sw[0], (unsigned)G, a.abortf);
+  // the slice in pairs; P threads per pair, each over every P-th partial, 16
+  // partials' loads in flight; then the P sums
+  const int S = (elems / 2 + G - 1) / G, e0 = g * S, len = max(0, min(S, elems / 2 - e0));
+  const int P = max(1, 256 / S), j = min(tid / S, P);
+  for (int x0 = 0; x0 < len; x0 += 256) {
+    const int x = x0 + (P > 1 ? tid - j * S : tid);
+    double2 sum = {0.0, 0.0};
+    if (x < len && (P == 1 || j < P)) {
+      const double2* src = reinterpret_cast<const double2*>(a.part) + e0 + x;
+      for (int q0 = (P > 1 ? j : 0); q0 < G; q0 += 16 * P) {
+        double2 v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = src[(size_t)min(q0 + u * P, G - 1) * (kBlkElems / 2)];
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+          if (q0 + u * P < G) {
+            sum.x += v[u].x;
+            sum.y += v[u].y;
+          }
+      }
     }
-    red[tid] = sum;
-    __syncthreads();
-    if (tid < len) {
-      double t = red[tid];
-      for (int q = 1; q < P; ++q) t += red[q * S + tid];
-      gs[e0 + tid] = t;
-    }
-  } else {
-    for (int x = tid; x < len; x += 256) {
-      const double* src = a.part + e0 + x;
-      double sum = 0.0;
-#pragma unroll 8
-      for (int q = 0; q < Gp; ++q) sum += src[(size_t)q * kCross];
-      gs[e0 + x] = sum;
+    double2* out = reinterpret_cast<double2*>(gs) + e0;
+    if (P == 1) {
+      if (x < len) out[x] = sum;
+    } else {
+      red[2 * tid] = sum.x;
+      red[2 * tid + 1] = sum.y;
+      __syncthreads();
+      if (tid < len) {
+        for (int q = 1; q < P; ++q) {
+          sum.x += red[2 * (q * S + tid)];
+          sum.y += red[2 * (q * S + tid) + 1];
+        }
+        out[tid] = sum;
+      }
     }
   }
   arrive(&sw[1], slot);
-}
-__device__ __forceinline__ void blk_wait(const CqrBlockArgs& a, int pass, int Hn) {
-  wait_count(&a.sync[pass * kBlkPassWords + 1], (unsigned)Hn, a.abortf);
-}
-template <int ELEMS>
-__device__ __forceinline__ void blk_allreduce(const CqrBlockArgs& a, int pass, bool contrib, int Gp, int hi, int Hn,
-                                              double* gs, double* red, int tid, unsigned* slot) {
-  blk_contribute<ELEMS>(a, pass, contrib, Gp, hi, Hn, gs, red, tid, slot);
-  blk_wait(a, pass, Hn);
+  wait_count(&sw[1], (unsigned)G, a.abortf);
 }
 
-// P = X^T Y over 64 rows (16 tiles of 16x16, tile t = 4 ti + tj, row-major).
-__device__ __forceinline__ void cross_partial(const double (*X)[LDA_S], const double (*Y)[LDA_S], double* out, int lane,
-                                              int wave) {
-  const int ti = wave;
+// This workgroup's partial Gram over its 64 rows: the 10 upper tiles of
+// X^T X, and for two halves the 16 of X^T Y and the 10 upper of Y^T Y.
+__device__ __forceinline__ void blk_gram(const double (*X)[LDA_S], const double (*Y)[LDA_S], bool two, double* out,
+                                         int lane, int wave) {
+  // Three tiles at a time per wave (their MFMAs independent of one another),
+  // every fourth tile from `wave` on; past the end, the last tile again.
+  const int nt = two ? 36 : 10;
+#pragma unroll 1
+  for (int t0 = wave; t0 < nt; t0 += 12) {
+    const double *xp[3], *yp[3];
+    f64x4 acc[3];
 #pragma unroll
-  for (int tj = 0; tj < 4; ++tj) {
-    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll 4
-    for (int k0 = 0; k0 < 64; k0 += 4) {
-      const double x = X[k0 + (lane >> 4)][16 * ti + (lane & 15)];
-      const double y = Y[k0 + (lane >> 4)][16 * tj + (lane & 15)];
-      acc = mfma16(x, y, acc);
+    for (int q = 0; q < 3; ++q) {
+      const int t = min(t0 + 4 * q, nt - 1);
+      int ti, tj;
+      tile_of(t < 10 ? t : t - 26, ti, tj);
+      const bool cross = t >= 10 && t < 26;
+      const int k = lane >> 4, c = lane & 15;
+      xp[q] = &(t < 26 ? X : Y)[k][16 * (cross ? (t - 10) >> 2 : ti) + c];
+      yp[q] = &(t < 10 ? X : Y)[k][16 * (cross ? (t - 10) & 3 : tj) + c];
+      acc[q] = f64x4{0.0, 0.0, 0.0, 0.0};
     }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) out[(4 * ti + tj) * 256 + ((lane >> 4) + 4 * r) * 16 + (lane & 15)] = acc[r];
-  }
-}
-
-__device__ __forceinline__ void load_tiles16(const double* gs, double (*M)[LDA_S], int tid) {
-  constexpr int Q = kCross / 256;
-  double v[Q];
-#pragma unroll
-  for (int q = 0; q < Q; ++q) v[q] = gs[tid + 256 * q];
-#pragma unroll
-  for (int q = 0; q < Q; ++q) {
-    const int e = tid + 256 * q;
-    const int t = e >> 8, r = (e >> 4) & 15, c = e & 15;
-    M[16 * (t >> 2) + r][16 * (t & 3) + c] = v[q];
-  }
-}
-
-// acc[tj] = row block `wave` of op(A) B, 64x64 full operands in LDS;
-// item r = C[16 wave + lane/16 + 4 r][16 tj + lane%16].
-template <bool TA>
-__device__ __forceinline__ void prod64(const double (*A)[LDA_S], const double (*B)[LDA_S], f64x4 (&acc)[4], int lane,
-                                       int wave) {
-#pragma unroll
-  for (int tj = 0; tj < 4; ++tj) {
-    acc[tj] = f64x4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll 4
+    for (int k0 = 0; k0 < 64; k0 += 4)
+#pragma unroll
+      for (int q = 0; q < 3; ++q) acc[q] = mfma16(xp[q][k0 * LDA_S], yp[q][k0 * LDA_S], acc[q]);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      if (t0 + 4 * q >= nt) continue;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) out[(t0 + 4 * q) * 256 + ((lane >> 4) + 4 * r) * 16 + (lane & 15)] = acc[q][r];
+    }
+  }
+}
+
+// The reduced Gram in registers: entry (tid / 16, tid % 16) of each tile.
+struct BlkGram {
+  double v[36];
+};
+__device__ __forceinline__ void read_gram(const double* gs, bool two, BlkGram& b, int tid) {
+#pragma unroll
+  for (int t = 0; t < 36; ++t) b.v[t] = (t < 10 || two) ? gs[t * 256 + tid] : 0.0;
+}
+
+// Largest |G - I| of it (NaN if any entry is); w columns.
+__device__ __forceinline__ double blk_dev(const BlkGram& b, int w, double* red4, int tid) {
+  const bool two = w > NB;
+  const int r = tid >> 4, c = tid & 15;
+  double d = 0.0;
+#pragma unroll
+  for (int t = 0; t < 36; ++t) {
+    if (t >= 10 && !two) break;
+    double want = 0.0;
+    if (t < 10 || t >= 26) {
+      int ti, tj;
+      tile_of(t < 10 ? t : t - 26, ti, tj);
+      if (ti == tj && r == c && 16 * ti + r + (t < 10 ? 0 : NB) < w) want = 1.0;
+    }
+    const double x = fabs(b.v[t] - want);
+    d = (x > d || x != x) ? x : d;
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    const double o = __shfl_xor(d, off, 64);
+    d = (o > d || o != o) ? o : d;
+  }
+  if ((tid & 63) == 0) red4[tid >> 6] = d;
+  __syncthreads();
+  double m = red4[0];
+#pragma unroll
+  for (int q = 1; q < 4; ++q) m = (red4[q] > m || red4[q] != red4[q]) ? red4[q] : m;
+  __syncthreads();
+  return m;
+}
+
+// M := the symmetric 64x64 block of the 10 tiles from T0 on, ones on the
+// diagonal beyond w columns.  Barrier after.
+template <int T0>
+__device__ __forceinline__ void put_gram(const BlkGram& b, double (*M)[LDA_S], int w, int tid) {
+  const int r = tid >> 4, c = tid & 15;
+#pragma unroll
+  for (int t = 0; t < 10; ++t) {
+    int ti, tj;
+    tile_of(t, ti, tj);
+    if (ti == tj && r > c) continue;  // one writer per entry of a diagonal tile
+    const double v = (ti == tj && r == c && 16 * ti + r >= w) ? 1.0 : b.v[T0 + t];
+    M[16 * ti + r][16 * tj + c] = v;
+    M[16 * tj + c][16 * ti + r] = v;
+  }
+  __syncthreads();
+}
+// M := G12.  Barrier after.
+__device__ __forceinline__ void put_cross(const BlkGram& b, double (*M)[LDA_S], int tid) {
+#pragma unroll
+  for (int t = 0; t < 16; ++t) M[16 * (t >> 2) + (tid >> 4)][16 * (t & 3) + (tid & 15)] = b.v[10 + t];
+  __syncthreads();
+}
+
+// acc[tj] = row block `wave` of op(A) op(B) over k in [0, klim), 64x64 operands in
+// LDS, op(X) = X^T with the flag; item r = C[16 wave + lane/16 + 4 r][16 tj + lane%16].
+// KB: op(B) is upper triangular, k < 16 (tj + 1).
+template <bool TA, bool TB = false, bool KB = false>
+__device__ __forceinline__ void prod64(const double (*A)[LDA_S], const double (*B)[LDA_S], int klim, f64x4 (&acc)[4],
+                                       int lane, int wave) {
+#pragma unroll
+  for (int tj = 0; tj < 4; ++tj) acc[tj] = f64x4{0.0, 0.0, 0.0, 0.0};
+  if constexpr (KB) {
+#pragma unroll
     for (int k0 = 0; k0 < 64; k0 += 4) {
       const int i = 16 * wave + (lane & 15), k = k0 + (lane >> 4);
       const double x = TA ? A[k][i] : A[i][k];
-      const double y = B[k][16 * tj + (lane & 15)];
-      acc[tj] = mfma16(x, y, acc[tj]);
+#pragma unroll
+      for (int tj = k0 / 16; tj < 4; ++tj) {
+        const int j = 16 * tj + (lane & 15);
+        acc[tj] = mfma16(x, TB ? B[j][k] : B[k][j], acc[tj]);
+      }
+    }
+    return;
+  }
+#pragma unroll 1
+  for (int kb = 0; kb < klim; kb += 16) {
+#pragma unroll
+    for (int k0 = 0; k0 < 16; k0 += 4) {
+      const int i = 16 * wave + (lane & 15), k = kb + k0 + (lane >> 4);
+      const double x = TA ? A[k][i] : A[i][k];
+#pragma unroll
+      for (int tj = 0; tj < 4; ++tj) {
+        const int j = 16 * tj + (lane & 15);
+        acc[tj] = mfma16(x, TB ? B[j][k] : B[k][j], acc[tj]);
+      }
     }
   }
 }
@@ -612,15 +747,37 @@ __device__ __forceinline__ void store_acc(const f64x4 (&acc)[4], double (*C)[LDA
 #pragma unroll
     for (int r = 0; r < 4; ++r) C[16 * wave + (lane >> 4) + 4 * r][16 * tj + (lane & 15)] = scale * acc[tj][r];
 }
+__device__ __forceinline__ void add_acc(const f64x4 (&acc)[4], double (*C)[LDA_S], double scale, int lane, int wave) {
+#pragma unroll
+  for (int tj = 0; tj < 4; ++tj)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) C[16 * wave + (lane >> 4) + 4 * r][16 * tj + (lane & 15)] += scale * acc[tj][r];
+}
+__device__ __forceinline__ void save_acc(const f64x4 (&acc)[4], double* dst, int lane, int wave) {
+#pragma unroll
+  for (int tj = 0; tj < 4; ++tj)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) dst[(16 * wave + (lane >> 4) + 4 * r) * NB + 16 * tj + (lane & 15)] = acc[tj][r];
+}
+__device__ __forceinline__ void save64(const double (*M)[LDA_S], double* dst, int tid) {
+  for (int e = tid; e < NB * NB; e += 256) dst[e] = M[e / NB][e % NB];
+}
 
-// Rejected block: all 128 columns column by column in place (team_factor),
-// the clean V, and T (128 x 128) from V's Gram by the recursion of
+// A uniform condition that the compiler must not pull out of a loop (loop
+// unswitching would give the loop's body, thousands of instructions, two copies).
+__device__ __forceinline__ bool one_copy(bool b) {
+  int v = __builtin_amdgcn_readfirstlane((int)b);
+  asm volatile("" : "+s"(v));
+  return v != 0;
+}
+
+// Rejected block: its w columns column by column in place (team_factor),
+// the clean V, and T from V's Gram by the recursion of
 // GenerateBlockTr("F","C") (Reflector.hpp:580-626), the Gram and T held in
 // scratch.  One workgroup; the others have left.
 __device__ __noinline__ void blk_refactor(CqrBlockArgs a, double* sh, int tid) {
-  constexpr int K = 2 * NB;
+  const int K = a.w, mp = a.mp;
   if (tid == 0) *a.fail = 1u;
-  const int mp = a.mp;
   double* Gm = a.scratch + kBG;
   double* Tm = a.scratch + kBTF;
   team_factor<double, 256, true>(mp, K, a.A, (int)a.lda, a.tau, sh);
@@ -655,46 +812,18 @@ __device__ __noinline__ void blk_refactor(CqrBlockArgs a, double* sh, int tid) {
   }
 }
 
-// The reconstruction's R = R2 R1 product (R1 from scratch at r1off) into acc;
-// M1 holds R2.
-__device__ __forceinline__ void blk_r_product(const double (*M1)[LDA_S], double (*M2)[LDA_S], const double* r1,
-                                              f64x4 (&acc)[4], int tid, int lane, int wave) {
-  load64(r1, M2, tid);
-  __syncthreads();
-  upper_product_row(M1, M2, false, nullptr, acc, lane, wave);
-}
-
-// T = -U D Z^T, Z = L^-1, from U/L packed in M1 and D in rowbuf (left there
-// by lu64); acc holds it (upper).  M2 is overwritten.
-__device__ __forceinline__ void blk_t_factor(const double (*M1)[LDA_S], double (*M2)[LDA_S], const double* rowbuf,
-                                             double* tmpb, f64x4 (&acc)[4], int tid, int lane, int wave) {
-  small64::inv_unit_lower64<LDA_S>(&M1[0][0], &M2[0][0], tmpb, tid);  // M2 = L^-1 (lower blocks)
-  upper_product_row<true>(M1, M2, true, rowbuf, acc, lane, wave);
+// T = -U D Z^T (upper) from U in M1 (on and above the diagonal), D in dcol and
+// Z = L^-1 in M2 (lower blocks); column `last` (no reflector) zero.
+__device__ __forceinline__ void blk_t_factor(const double (*M1)[LDA_S], const double (*M2)[LDA_S], const double* dcol,
+                                             int last, f64x4 (&acc)[4], int lane, int wave) {
+  upper_product_row<true>(M1, M2, true, dcol, acc, lane, wave);
 #pragma unroll
   for (int tj = 0; tj < 4; ++tj)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = 16 * wave + (lane >> 4) + 4 * r, j = 16 * tj + (lane & 15);
-      acc[tj][r] = (i <= j) ? -acc[tj][r] : 0.0;
+      acc[tj][r] = (i <= j && j != last) ? -acc[tj][r] : 0.0;
     }
-}
-
-// R2 and R2^-1 from the second pass's Gram in M1 (dev <= kSecondPass):
-// first order when |E| <= 2^-40, factored otherwise.
-__device__ __forceinline__ void blk_second_r(double (*M1)[LDA_S], double (*M2)[LDA_S], double dev, double* tmpb,
-                                             double* gdiag, int* okf, int tid) {
-  if (dev <= kFirstOrder) {
-    for (int e = tid; e < NB * NB; e += 256) {
-      const int i = e / NB, j = e % NB;
-      const double E = M1[i][j] - (i == j ? 1.0 : 0.0);
-      const double eu = (i < j) ? E : ((i == j) ? 0.5 * E : 0.0);
-      M1[i][j] = (i == j ? 1.0 : 0.0) + eu;
-      M2[i][j] = (i == j ? 1.0 : 0.0) - eu;
-    }
-    __syncthreads();
-  } else {
-    small64::chol64<LDA_S>(&M1[0][0], &M2[0][0], tmpb, gdiag, okf, tid);
-  }
 }
 
 }  // namespace
@@ -715,11 +844,12 @@ __global__ __launch_bounds__(256) void cqr_block_kernel(CqrBlockArgs a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = blockIdx.x, G = gridDim.x;
   const int r0 = 64 * g;
-  const int mp = a.mp;
+  const int mp = a.mp, w = a.w, w2 = w - NB;  // w2: columns of the second half
+  const bool two = w2 > 0;
   double* sc = a.scratch;
-  double* part = a.part + (size_t)g * kCross;
+  double* part = a.part + (size_t)g * kBlkElems;
 
-  // Both panels' rows of this workgroup.
+  // Both halves' rows of this workgroup, zero outside the block.
   {
     constexpr int PER = 64 * NB / 256;
     double v[2][PER];
@@ -727,8 +857,8 @@ __global__ __launch_bounds__(256) void cqr_block_kernel(CqrBlockArgs a) {
     for (int q = 0; q < PER; ++q) {
       const int e = tid + 256 * q, r = e % 64, c = e / 64;
       const bool in = r0 + r < mp;
-      v[0][q] = in ? a.A[(size_t)(r0 + r) + (size_t)c * a.lda] : 0.0;
-      v[1][q] = in ? a.A[(size_t)(r0 + r) + (size_t)(c + NB) * a.lda] : 0.0;
+      v[0][q] = (in && c < w) ? a.A[(size_t)(r0 + r) + (size_t)c * a.lda] : 0.0;
+      v[1][q] = (in && c < w2) ? a.A[(size_t)(r0 + r) + (size_t)(c + NB) * a.lda] : 0.0;
     }
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
@@ -739,244 +869,265 @@ __global__ __launch_bounds__(256) void cqr_block_kernel(CqrBlockArgs a) {
   }
   __syncthreads();
 
-  // ---- Panel 1 ----
-  gram_partial<64>(Ab1, part, lane, wave);
-  blk_allreduce<kGramElems>(a, 0, true, G, g, G, a.gsum, tmpb, tid, &slot);
-  load_gram(a.gsum, M1, tid);
-  __syncthreads();
-  if (!small64::chol64<LDA_S>(&M1[0][0], &M2[0][0], tmpb, gdiag, &okf, tid)) {
-    if (g == 0) blk_refactor(a, rowbuf, tid);
-    return;
-  }
-  if (g == 1)
-    for (int e = tid; e < NB * NB; e += 256) sc[kBR1a + e] = M1[e / NB][e % NB];
-  times_upper<64>(Ab1, M2, lane, wave);
-  gram_partial<64>(Ab1, part, lane, wave);
-  blk_allreduce<kGramElems>(a, 1, true, G, g, G, a.gsum + kCross, tmpb, tid, &slot);
-  load_gram(a.gsum + kCross, M1, tid);
-  __syncthreads();
-  double dev = dev_from_identity(M1, red4, tid);
-  if (!(dev <= kSecondPass)) {
-    if (g == 0) blk_refactor(a, rowbuf, tid);
-    return;
-  }
-  blk_second_r(M1, M2, dev, tmpb, gdiag, &okf, tid);
-  times_upper<64>(Ab1, M2, lane, wave);  // Ab1 = Q, M1 = R2
-  if (g == 0) {
-    for (int e = tid; e < NB * NB; e += 256) M1[e / NB][e % NB] = Ab1[e / NB][e % NB];
-    __syncthreads();
-    small64::lu64<LDA_S>(&M1[0][0], rowbuf, &M2[0][0], tmpb, tid);  // M1 = U and L, M2 = U^-1
-    for (int e = tid; e < NB * NB; e += 256) sc[kBU1i + e] = M2[e / NB][e % NB];
-    if (tid < NB) {
-      sc[kBD1 + tid] = rowbuf[tid];
-      sc[kBTau1 + tid] = -M1[tid][tid] * rowbuf[tid];
+  // ---- 1 and 2: passes; workgroup 2 keeps their factors for R ----
+  int np = 0;  // passes done (factors at sc + kBR + 3 * 4096 * pass)
+#pragma unroll 1
+  for (int pass = 0;; ++pass) {
+    blk_gram(Ab1, Ab2, two, part, lane, wave);
+    double* gs = a.gsum + (size_t)pass * kBlkElems;
+    blk_allreduce(a, two ? kBlkElems : kGramElems, pass, g, G, gs, tmpb, tid, &slot);
+    BlkGram gm;
+    read_gram(gs, two, gm, tid);
+    double dev = 1.0;
+    if (pass > 0) dev = blk_dev(gm, w, red4, tid);
+    double* rp = sc + kBR + (size_t)3 * 4096 * pass;
+    const bool is_first = pass > 0 && dev <= kFirstOrder;
+    bool ok = pass == 0 || (dev <= kThirdPass && (is_first || pass < kBlkPasses));
+#pragma unroll 1
+    for (int half = 0; half < (two ? 2 : 1) && ok; ++half) {
+      const bool first = one_copy(is_first), second_half = one_copy(half != 0), keep = one_copy(g == 2);
+      double(*X)[LDA_S] = second_half ? M2 : M1;   // the Gram, then R
+      double(*Xi)[LDA_S] = second_half ? M1 : M2;  // R^-1
+      f64x4 acc[4];
+      if (!second_half) {
+        put_gram<0>(gm, M1, w, tid);
+        if (tid < NB) gdiag[tid] = M1[tid][tid];
+      } else {
+        put_cross(gm, M1, tid);
+        if (!first) {
+          prod64<true>(M2, M1, 16 * (wave + 1), acc, lane, wave);  // R12 = R11^-T G12 (first order: E12)
+          __syncthreads();
+          store_acc(acc, M1, 1.0, lane, wave);
+        }
+        put_gram<26>(gm, M2, w2, tid);  // its barrier: M1 is complete too
+        if (keep) save64(M1, rp + 4096, tid);
+        prod64<false>(Ab1, M1, 64, acc, lane, wave);
+        add_acc(acc, Ab2, -1.0, lane, wave);  // A2 - Q1 R12
+        if (!first) {
+          if (tid < NB) gdiag[tid] = M2[tid][tid];  // the columns' own norms
+          prod64<true>(M1, M1, 64, acc, lane, wave);
+          __syncthreads();
+          add_acc(acc, M2, -1.0, lane, wave);  // G22 - R12^T R12
+        }
+        __syncthreads();
+      }
+      double* rs = rp + (second_half ? 8192 : 0);
+      if (first) {
+        // R = I + S, R^-1 = I - S with S = triu(E) - diag(E)/2
+        for (int e = tid; e < NB * NB; e += 256) {
+          const int i = e / NB, c = e % NB;
+          const double one = (i == c) ? 1.0 : 0.0, E = X[i][c] - one, S = (i < c) ? E : 0.5 * one * E;
+          Xi[i][c] = one - S;
+          if (keep) rs[e] = one + S;
+        }
+        __syncthreads();
+      } else {
+        ok = small64::chol64<LDA_S>(&X[0][0], &Xi[0][0], tmpb, gdiag, &okf, tid);
+        if (ok && keep)
+          for (int e = tid; e < NB * NB; e += 256) rs[e] = (e / NB <= e % NB) ? X[e / NB][e % NB] : 0.0;
+      }
+      if (ok) times_upper<64>(second_half ? Ab2 : Ab1, Xi, lane, wave);
     }
-    publish(&a.sync[kBlkPub1]);
-    for (int e = tid; e < NB * NB; e += 256) {
-      const int i = e / NB, j = e % NB;
-      Ab1[i][j] = (i > j) ? M1[i][j] : (i == j ? 1.0 : 0.0);  // V1's top block: L1
+    if (!ok) {
+      if (g == 0) blk_refactor(a, rowbuf, tid);
+      return;
+    }
+    np = pass + 1;
+    if (pass > 0 && dev <= kSecondPass) break;  // orthonormal to working precision now
+  }
+
+  // ---- 3: reconstruction ----
+  const int last = (mp == w) ? w - 1 : -1;  // the column without a reflector
+  const double pmax = a.zero_tails ? 1.0 - 0x1p-40 : 2.0;
+  f64x4 racc[3][4];
+  if (g == 2) {
+    // R's product of the passes' factors, in place of the first one's
+    double* c0 = sc + kBR;
+    for (int p = 1; p < np; ++p) {
+      const double* rp = sc + kBR + (size_t)3 * 4096 * p;
+      __syncthreads();
+      load64(rp, M1, tid);
+      load64(c0, M2, tid);
+      __syncthreads();
+      upper_product_row(M1, M2, false, nullptr, racc[0], lane, wave);
+      if (two) {
+        __syncthreads();
+        load64(c0 + 4096, M2, tid);
+        __syncthreads();
+        prod64<false>(M1, M2, 64, racc[1], lane, wave);
+        __syncthreads();
+        load64(rp + 4096, M1, tid);
+        load64(c0 + 8192, M2, tid);
+        __syncthreads();
+        f64x4 x[4];
+        prod64<false, false, true>(M1, M2, 64, x, lane, wave);
+#pragma unroll
+        for (int tj = 0; tj < 4; ++tj) racc[1][tj] += x[tj];
+        __syncthreads();
+        load64(rp + 8192, M1, tid);
+        __syncthreads();
+        upper_product_row(M1, M2, false, nullptr, racc[2], lane, wave);
+      }
+      if (p + 1 < np) {
+        __syncthreads();
+        save_acc(racc[0], c0, lane, wave);
+        if (two) {
+          save_acc(racc[1], c0 + 4096, lane, wave);
+          save_acc(racc[2], c0 + 8192, lane, wave);
+        }
+      }
     }
     __syncthreads();
-  } else {
-    f64x4 racc[4];
-    if (g == 1) blk_r_product(M1, M2, sc + kBR1a, racc, tid, lane, wave);
-    wait_flag(&a.sync[kBlkPub1], a.abortf);
-    if (g == 1) {
+  }
+#pragma unroll 1
+  for (int half = 0; half < (two ? 2 : 1); ++half) {
+    const bool sh = one_copy(half != 0), mine = one_copy(g == half), fh = one_copy(two && half == 0);
+    double(*Ab)[LDA_S] = sh ? Ab2 : Ab1;
+    unsigned* pub = &a.sync[sh ? kBlkPub2 : kBlkPub1];
+    double* ui = sc + (sh ? kBU2i : kBU1i);
+    double* dd = sc + (sh ? kBD2 : kBD1);
+    const int o = sh ? NB : 0, wh = min(w - o, NB);                 // this half's first column, its width
+    const int lasth = (last >= o && last < o + NB) ? last - o : -1;  // its column without a reflector
+    f64x4 acc[4];
+    if (mine) {
+      for (int e = tid; e < NB * NB; e += 256) M1[e / NB][e % NB] = Ab[e / NB][e % NB];
+      __syncthreads();
+      // M1 = U and L, M2 = U^-1
+      const bool fits = small64::lu64<LDA_S>(&M1[0][0], rowbuf, &M2[0][0], tmpb, &okf, tid, lasth, pmax);
+      save64(M2, ui, tid);
+      if (tid < NB) dd[tid] = rowbuf[tid];
+      publish(pub, fits ? 1u : kRejected);
+      if (!fits) {
+        if (g == 0) blk_refactor(a, rowbuf, tid);
+        return;
+      }
+      for (int e = tid; e < NB * NB; e += 256) {
+        const int i = e / NB, j = e % NB;
+        const double v = (i > j) ? M1[i][j] : (i == j ? 1.0 : 0.0);
+        if (!sh) Ab1[i][j] = v;  // V1's top block: L11
+        else M1[i][j] = (i > j) ? v : M1[i][j];
+      }
+      if (tid < wh) a.tau[o + tid] = (tid == lasth) ? 0.0 : -M1[tid][tid] * rowbuf[tid];
+      __syncthreads();
+      small64::inv_unit_lower64<LDA_S>(&M1[0][0], &M2[0][0], tmpb, tid);  // M2 = L^-1 (lower blocks)
+      if (fh) {
+        prod64<false>(M2, Ab2, 16 * (wave + 1), acc, lane, wave);  // U12 = L11^-1 Q2(0:64)
+        save_acc(acc, sc + kBU12, lane, wave);
+        publish(&a.sync[kBlkPubU12]);
+      }
+      blk_t_factor(M1, M2, rowbuf, lasth, acc, lane, wave);
+      if (fh) {
+        save_acc(acc, sc + kBT1, lane, wave);
+        publish(&a.sync[kBlkPubT1]);
+      }
 #pragma unroll
       for (int tj = 0; tj < 4; ++tj)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int i = 16 * wave + (lane >> 4) + 4 * r, j = 16 * tj + (lane & 15);
-          sc[kBRF1 + i * NB + j] = sc[kBD1 + i] * racc[tj][r];
+          a.T[(size_t)(o + i) + (size_t)(o + j) * a.ldt] = acc[tj][r];
         }
-    }
-    __syncthreads();
-    load64(sc + kBU1i, M2, tid);
-    __syncthreads();
-    times_upper<64>(Ab1, M2, lane, wave);  // Ab1 = V1 rows
-  }
-
-  // ---- Panel 1's reflectors applied to panel 2: A2 -= V1 (T1^T (V1^T A2)) ----
-  cross_partial(Ab1, Ab2, part, lane, wave);
-  blk_contribute<kCross>(a, 2, true, G, g - 1, G - 1, a.gsum + 2 * kCross, tmpb, tid, &slot);  // g0: T1
-  if (g == 0) {
-    // T1 while the reduction completes; the LU is still in M1 and rowbuf.
-    f64x4 tacc[4];
-    blk_t_factor(M1, M2, rowbuf, tmpb, tacc, tid, lane, wave);
-#pragma unroll
-    for (int tj = 0; tj < 4; ++tj)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = 16 * wave + (lane >> 4) + 4 * r, j = 16 * tj + (lane & 15);
-        sc[kBT1 + i * NB + j] = tacc[tj][r];
-        a.T[(size_t)i + (size_t)j * a.ldt] = tacc[tj][r];
+      // A only once the second half is accepted too
+      if (fh && wait_verdict(&a.sync[kBlkPub2], a.abortf, &slot) == kRejected) {
+        blk_refactor(a, rowbuf, tid);
+        return;
       }
-    publish(&a.sync[kBlkPubT1]);
-  }
-  blk_wait(a, 2, G - 1);
-  wait_flag(&a.sync[kBlkPubT1], a.abortf);
-  load_tiles16(a.gsum + 2 * kCross, M2, tid);                                     // W
-  load64(sc + kBT1, M1, tid);  // T1
-  __syncthreads();
-  {
-    f64x4 acc[4];
-    prod64<true>(M1, M2, acc, lane, wave);  // Z = T1^T W
-    __syncthreads();
-    store_acc(acc, M1, 1.0, lane, wave);
-    __syncthreads();
-    prod64<false>(Ab1, M1, acc, lane, wave);  // V1 Z
-#pragma unroll
-    for (int tj = 0; tj < 4; ++tj)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) Ab2[16 * wave + (lane >> 4) + 4 * r][16 * tj + (lane & 15)] -= acc[tj][r];
-    __syncthreads();
-  }
-
-  // ---- Panel 2: rows 64.. (workgroups 1..), LU and T by workgroup 1, R by 2 ----
-  const bool p2 = (g >= 1);
-  const int gi = g - 1, G2 = G - 1;
-  if (p2) gram_partial<64>(Ab2, a.part + (size_t)gi * kCross, lane, wave);
-  blk_allreduce<kGramElems>(a, 3, p2, G2, g, G, a.gsum + 3 * kCross, tmpb, tid, &slot);
-  load_gram(a.gsum + 3 * kCross, M1, tid);
-  __syncthreads();
-  if (!small64::chol64<LDA_S>(&M1[0][0], &M2[0][0], tmpb, gdiag, &okf, tid)) {
-    if (g == 0) blk_refactor(a, rowbuf, tid);
-    return;
-  }
-  if (g == 2)
-    for (int e = tid; e < NB * NB; e += 256) sc[kBR1b + e] = M1[e / NB][e % NB];
-  if (p2) times_upper<64>(Ab2, M2, lane, wave);
-  else __syncthreads();
-  if (p2) gram_partial<64>(Ab2, a.part + (size_t)gi * kCross, lane, wave);
-  blk_allreduce<kGramElems>(a, 4, p2, G2, g, G, a.gsum + 4 * kCross, tmpb, tid, &slot);
-  load_gram(a.gsum + 4 * kCross, M1, tid);
-  __syncthreads();
-  dev = dev_from_identity(M1, red4, tid);
-  if (!(dev <= kSecondPass)) {
-    if (g == 0) blk_refactor(a, rowbuf, tid);
-    return;
-  }
-  blk_second_r(M1, M2, dev, tmpb, gdiag, &okf, tid);
-
-  // Both panels are accepted: panel 1's results go out now.
-  if (g == 0) {
-    for (int e = tid; e < NB * NB; e += 256) {
-      const int i = e % NB, j = e / NB;
-      const double v = Ab1[i][j];
-      if (i > j) a.A[(size_t)i + (size_t)j * a.lda] = v;
-      a.V[(size_t)i + (size_t)j * a.ldv] = v;
-      a.A[(size_t)i + (size_t)(j + NB) * a.lda] = Ab2[i][j];  // R12
-      a.V[(size_t)i + (size_t)(j + NB) * a.ldv] = 0.0;
-      a.T[(size_t)(i + NB) + (size_t)j * a.ldt] = 0.0;
-    }
-    if (tid < NB) a.tau[tid] = sc[kBTau1 + tid];
-  } else {
-    for (int e = tid; e < 64 * NB; e += 256) {
-      const int r = e % 64, c = e / 64, gr = r0 + r;
-      if (gr < mp) {
-        const double v = Ab1[r][c];
-        a.A[(size_t)gr + (size_t)c * a.lda] = v;
-        a.V[(size_t)gr + (size_t)c * a.ldv] = v;
-      }
-    }
-    if (g == 1)
       for (int e = tid; e < NB * NB; e += 256) {
         const int i = e % NB, j = e / NB;
-        if (i <= j) a.A[(size_t)i + (size_t)j * a.lda] = sc[kBRF1 + i * NB + j];
+        const double l = M1[i][j];
+        if (o + i < mp && j < wh) {
+          if (i > j) a.A[(size_t)(o + i) + (size_t)(o + j) * a.lda] = l;
+          a.V[(size_t)(o + i) + (size_t)(o + j) * a.ldv] = (i > j) ? l : (i == j ? 1.0 : 0.0);
+        }
+        if (!sh) {
+          if (j < w2) a.V[(size_t)i + (size_t)(j + NB) * a.ldv] = 0.0;
+          if (fh) a.T[(size_t)(i + NB) + (size_t)j * a.ldt] = 0.0;
+        } else if (NB + i < mp) {
+          const double v = Ab1[i][j];
+          a.A[(size_t)(NB + i) + (size_t)j * a.lda] = v;
+          a.V[(size_t)(NB + i) + (size_t)j * a.ldv] = v;
+        }
       }
-  }
-
-  if (p2) times_upper<64>(Ab2, M2, lane, wave);  // Ab2 = Q2 (g >= 1), M1 = R2'
-  else __syncthreads();
-  if (g == 1) {
-    for (int e = tid; e < NB * NB; e += 256) M1[e / NB][e % NB] = Ab2[e / NB][e % NB];
-    __syncthreads();
-    small64::lu64<LDA_S>(&M1[0][0], rowbuf, &M2[0][0], tmpb, tid);
-    for (int e = tid; e < NB * NB; e += 256) sc[kBU2i + e] = M2[e / NB][e % NB];
-    if (tid < NB) sc[kBD2 + tid] = rowbuf[tid];
-    publish(&a.sync[kBlkPub2]);
-    for (int e = tid; e < NB * NB; e += 256) {
-      const int i = e % NB, j = e / NB;
-      const double l = M1[i][j];
-      const double v = (i > j) ? l : (i == j ? 1.0 : 0.0);
-      Ab2[i][j] = v;
-      if (i > j) a.A[(size_t)(NB + i) + (size_t)(NB + j) * a.lda] = l;
-      a.V[(size_t)(NB + i) + (size_t)(NB + j) * a.ldv] = v;
-    }
-    if (tid < NB) a.tau[NB + tid] = -M1[tid][tid] * rowbuf[tid];
-    __syncthreads();
-  } else if (g >= 2) {
-    f64x4 racc[4];
-    if (g == 2) blk_r_product(M1, M2, sc + kBR1b, racc, tid, lane, wave);
-    wait_flag(&a.sync[kBlkPub2], a.abortf);
-    if (g == 2) {
+      if (!sh) return;
+      // T12 = -(T11 L21^T + U12 D2) L22^-T
+      wait_flag(&a.sync[kBlkPubT1], a.abortf);  // its barrier: M1 is free
+      load64(sc + kBT1, M1, tid);
+      __syncthreads();
+      prod64<false, true>(M1, Ab1, 64, acc, lane, wave);
+      __syncthreads();
 #pragma unroll
       for (int tj = 0; tj < 4; ++tj)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int i = 16 * wave + (lane >> 4) + 4 * r, j = 16 * tj + (lane & 15);
-          if (i <= j) a.A[(size_t)(NB + i) + (size_t)(NB + j) * a.lda] = sc[kBD2 + i] * racc[tj][r];
+          M1[i][j] = acc[tj][r] + sc[kBU12 + i * NB + j] * rowbuf[j];
         }
+      __syncthreads();
+      prod64<false, true, true>(M1, M2, 64, acc, lane, wave);
+#pragma unroll
+      for (int tj = 0; tj < 4; ++tj)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = 16 * wave + (lane >> 4) + 4 * r, j = 16 * tj + (lane & 15);
+          a.T[(size_t)i + (size_t)(NB + j) * a.ldt] = (j == lasth) ? 0.0 : -acc[tj][r];
+        }
+      return;
     }
+    if (g < half) return;  // (workgroup 0 left above)
+    if (wait_verdict(pub, a.abortf, &slot) == kRejected) return;
+    load64(ui, M2, tid);
     __syncthreads();
-    load64(sc + kBU2i, M2, tid);
-    __syncthreads();
-    times_upper<64>(Ab2, M2, lane, wave);  // V2 rows
-    for (int e = tid; e < 64 * NB; e += 256) {
-      const int r = e % 64, c = e / 64, gr = r0 + r;
-      if (gr < mp) {
-        const double v = Ab2[r][c];
-        a.A[(size_t)gr + (size_t)(c + NB) * a.lda] = v;
-        a.V[(size_t)gr + (size_t)(c + NB) * a.ldv] = v;
-      }
+    times_upper<64>(Ab, M2, lane, wave);  // V rows of this half
+    if (fh) {
+      wait_flag(&a.sync[kBlkPubU12], a.abortf);
+      load64(sc + kBU12, M1, tid);
+      __syncthreads();
+      prod64<false>(Ab1, M1, 64, acc, lane, wave);
+      add_acc(acc, Ab2, -1.0, lane, wave);  // Q2 - V1 U12
+      __syncthreads();
     }
   }
-
-  // ---- Merge: T12 = -T1 (V1^T V2) T2, by workgroup 1 (which holds LU2) ----
-  if (!p2) return;
-  cross_partial(Ab1, Ab2, a.part + (size_t)gi * kCross, lane, wave);
-  blk_contribute<kCross>(a, 5, true, G2, g - 2, G - 2, a.gsum + 5 * kCross, tmpb, tid, &slot);  // g1: T2
-  if (g != 1) return;
-  {
-    f64x4 tacc[4];
-    blk_t_factor(M1, M2, rowbuf, tmpb, tacc, tid, lane, wave);  // T2
+  for (int e = tid; e < 64 * NB; e += 256) {
+    const int r = e % 64, c = e / 64, gr = r0 + r;
+    if (gr < mp && c < w) {
+      const double v = Ab1[r][c];
+      a.A[(size_t)gr + (size_t)c * a.lda] = v;
+      a.V[(size_t)gr + (size_t)c * a.ldv] = v;
+    }
+    if (gr < mp && c < w2) {
+      const double v = Ab2[r][c];
+      a.A[(size_t)gr + (size_t)(c + NB) * a.lda] = v;
+      a.V[(size_t)gr + (size_t)(c + NB) * a.ldv] = v;
+    }
+  }
+  if (g == 2) {
 #pragma unroll
     for (int tj = 0; tj < 4; ++tj)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int i = 16 * wave + (lane >> 4) + 4 * r, j = 16 * tj + (lane & 15);
-        a.T[(size_t)(NB + i) + (size_t)(NB + j) * a.ldt] = tacc[tj][r];
+        if (i <= j && j < w) a.A[(size_t)i + (size_t)j * a.lda] = sc[kBD1 + i] * racc[0][tj][r];
+        if (j < w2) {
+          a.A[(size_t)i + (size_t)(NB + j) * a.lda] = sc[kBD1 + i] * racc[1][tj][r];
+          if (i <= j) a.A[(size_t)(NB + i) + (size_t)(NB + j) * a.lda] = sc[kBD2 + i] * racc[2][tj][r];
+        }
       }
-    store_acc(tacc, Ab2, 1.0, lane, wave);  // Ab2 was last read before the arrival's barrier
   }
-  blk_wait(a, 5, G - 2);
-  load_tiles16(a.gsum + 5 * kCross, M2, tid);                                     // S
-  load64(sc + kBT1, M1, tid);  // T1
-  __syncthreads();
-  f64x4 acc[4];
-  prod64<false>(M1, M2, acc, lane, wave);  // X = T1 S
-  __syncthreads();
-  store_acc(acc, M1, 1.0, lane, wave);
-  __syncthreads();
-  prod64<false>(M1, Ab2, acc, lane, wave);  // X T2
-#pragma unroll
-  for (int tj = 0; tj < 4; ++tj)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = 16 * wave + (lane >> 4) + 4 * r, j = 16 * tj + (lane & 15);
-      a.T[(size_t)i + (size_t)(NB + j) * a.ldt] = -acc[tj][r];
-    }
 }
 
-int cqr_block_groups(int mp, int max_groups) {
-  if (mp < 3 * NB) return 0;
-  const int G = (mp + 63) / 64;
-  return (G >= 3 && G <= max_groups && G <= 16 * kGroup) ? G : 0;
+int cqr_block_groups(int mp, int w, int max_groups) {
+  // Fewer than 16 columns, in the first half or beyond it, are left to the
+  // column-wise panel: the launch costs 108 us for one half and 230 for two at
+  // any width up to 1000 rows, that panel 5 to 7 us a column (16 columns: 108 us
+  // at 250 rows, 134 at 1000, 147 at 8000 against 138 here).
+  if (w < 16 || (w > NB && w < NB + 16) || w > 2 * NB || mp < w) return 0;
+  const int G = std::max(3, (mp + 63) / 64);  // the roles of three workgroups
+  return (G <= max_groups && G <= 16 * kGroup) ? G : 0;
 }
 
 hipError_t launch_cqr_block(const CqrBlockArgs& a, int G, hipStream_t st) {
-  if (G < 3 || (long)G * 64 < a.mp || (long)(G - 1) * 64 >= a.mp || a.lda < a.mp || a.ldv < a.mp || a.ldt < 2 * NB ||
-      !a.fail || !a.sync || !a.abortf)
+  if (a.w < 1 || a.w > 2 * NB || a.mp < a.w || G < 3 || (long)G * 64 < a.mp || (G > 3 && (long)(G - 1) * 64 >= a.mp) ||
+      a.lda < a.mp || a.ldv < a.mp || a.ldt < 2 * NB || !a.fail || !a.sync || !a.abortf)
     return hipErrorInvalidValue;
   hipLaunchKernelGGL(cqr_block_kernel, dim3(G), dim3(256), 0, st, a);
   return hipGetLastError();

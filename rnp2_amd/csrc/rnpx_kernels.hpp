@@ -77,12 +77,12 @@ __device__ __forceinline__ unsigned arrive(unsigned* counter, unsigned* slot) {
 }
 
 // Set a flag after all the workgroup's global stores are done.
-__device__ __forceinline__ void publish(unsigned* flag) {
+__device__ __forceinline__ void publish(unsigned* flag, unsigned value = 1u) {
   wait_stores();
   __syncthreads();
   if (threadIdx.x == 0) {
     release_agent();
-    __hip_atomic_store(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(flag, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -248,22 +248,22 @@ constexpr int kCqrMaxGroups = 256;
 int cqr_panel_groups(int mp, int max_groups, int* rw);
 hipError_t launch_cqr_panel(const CqrArgs& a, int G, int rw, hipStream_t st);
 
-// A real outer block of 128 columns (two 64-column panels) in one launch
-// (rnpx_cqr.hip): both panels by CholeskyQR2 + reconstruction, panel 1
-// applied to panel 2 and the compact-WY forms merged in LDS.  Outputs: R and
-// V packed in A (128 columns), tau (128), the block's clean V (ldv >= mp,
-// zeros above the second panel) and T (128 x 128, ldt >= 128).  If either
-// panel is rejected, A is untouched until workgroup 0 refactors the block
-// column by column in the same launch (*fail = 1).  G = ceil(mp/64)
-// workgroups, all resident at once (they meet at grid-wide reductions).
+// A real outer block of w <= 128 columns in one launch (rnpx_cqr.hip) by
+// CholeskyQR2 and Householder reconstruction.  Outputs: R and V packed in A,
+// tau (w), the block's clean V (ldv >= mp, zeros above the second 64 columns)
+// and T (w x w; 128 columns of ldt >= 128 are written).  If the block is
+// rejected, A is untouched until workgroup 0 refactors it column by column in
+// the same launch (*fail = 1).  G workgroups of 64 rows, at least three, all
+// resident at once (they meet at grid-wide reductions).
 struct CqrBlockArgs {
-  int mp;               // block rows (>= 192)
+  int mp, w;            // block rows and columns (w <= 128, w <= mp)
+  bool zero_tails;      // columns with exact zeros below the diagonal get tau = 0 (column by column)
   double* A; long lda;  // block top-left
-  double* tau;          // out: 128 scalars
-  double* V; long ldv;  // out: clean V, mp x 128
-  double* T; long ldt;  // out: 128 x 128 T
-  double* part;         // scratch: G * 4096 (each workgroup's partial products)
-  double* gsum;         // scratch: 6 * 4096 (reduced products of each pass)
+  double* tau;          // out: w scalars
+  double* V; long ldv;  // out: clean V, mp x w
+  double* T; long ldt;  // out: T
+  double* part;         // scratch: G * kCqrBlockPart (each workgroup's partial Gram)
+  double* gsum;         // scratch: 4 * kCqrBlockPart (the reduced Gram of each pass)
   double* scratch;      // scratch: kCqrBlockScratch doubles
   unsigned* sync;       // kCqrBlockSyncWords words, zero at launch
   unsigned* abortf;     // sticky error flag
@@ -271,8 +271,9 @@ struct CqrBlockArgs {
 };
 constexpr int kCqrBlockSyncWords = 256;
 constexpr int kCqrBlockScratch = 65728;
-// Workgroups for an mp-row block, 0 when the block kernel does not apply.
-int cqr_block_groups(int mp, int max_groups);
+constexpr int kCqrBlockPart = 36 * 256;  // the upper 16 x 16 tiles of a 128 x 128 Gram
+// Workgroups for an mp-row, w-column block, 0 when the block kernel does not apply.
+int cqr_block_groups(int mp, int w, int max_groups);
 hipError_t launch_cqr_block(const CqrBlockArgs& a, int G, hipStream_t st);
 // Waits (bounded) until the G workgroups of the block kernel with these sync
 // words have all started.

@@ -688,17 +688,23 @@ int geqrf_dev(Handle* h, int m, int n, T* A, long lda, T* tau, T* B, int nrhs, l
   RNPX_TRY(h->gram.ensure(sizeof(T) * (size_t)nb * nb, h));
   RNPX_TRY(h->ppart.ensure(sizeof(T) * 2 * (size_t)kMaxPanelGroups * nb + 64, h));
   RNPX_TRY(h->rowbuf.ensure(sizeof(T) * 2 * (size_t)nb, h));
-  const int sync_words = 1 + 2 * npan + kCqrSyncWords * npan;
+  // (one panel's words more: a last block of one panel still uses two)
+  const int sync_words = 1 + 2 * npan + kCqrSyncWords * (npan + 1);
   RNPX_TRY(h->sync.ensure(sizeof(unsigned) * (size_t)sync_words, h));
   // Outer blocks in one launch (real, 64-column panels, 128-column blocks,
-  // tuning panel 0): buffers for the block kernel.
-  const bool use_block = !S<T>::cplx && h->tune.panel == 0 && nb == 64 && nbo % (2 * nb) == 0 &&
-                         cqr_block_groups(m, std::min(256, h->num_cus)) > 0;
+  // tuning panel 0): buffers for the block kernel (without room for them in the
+  // handle's budget: panel by panel).
+  bool use_block = !S<T>::cplx && h->tune.panel == 0 && nb == 64 && nbo % (2 * nb) == 0 &&
+                         cqr_block_groups(m, std::min(nb, k), std::min(256, h->num_cus)) > 0;
   static_assert(2 * kCqrSyncWords >= kCqrBlockSyncWords, "a block uses its two panels' sync words");
   if (use_block) {
-    RNPX_TRY(h->cqr_part.ensure(sizeof(double) * (size_t)cqr_block_groups(m, std::min(256, h->num_cus)) * 4096, h));
-    RNPX_TRY(h->cqr_gsum.ensure(sizeof(double) * 6 * 4096, h));
-    RNPX_TRY(h->cqr_scratch.ensure(sizeof(double) * kCqrBlockScratch, h));
+    const std::pair<Buffer*, size_t> need[] = {
+        {&h->cqr_part, sizeof(double) * (size_t)std::max(3, (m + 63) / 64) * kCqrBlockPart},
+        {&h->cqr_gsum, sizeof(double) * 4 * kCqrBlockPart},
+        {&h->cqr_scratch, sizeof(double) * kCqrBlockScratch}};
+    const int s = reserve(h, need, 3);
+    if (s == RNPX_ERR_NOMEM) use_block = false;
+    else if (s) return s;
   }
   {
     int g0 = 0, rw0 = 0;
@@ -735,7 +741,7 @@ int geqrf_dev(Handle* h, int m, int n, T* A, long lda, T* tau, T* B, int nrhs, l
 
   // Columns [i, i + w) (rows [i, m)) factored into V (row 0 = row i,
   // leading dimension ldv) and T (ldt) on stream ps: one block-kernel launch
-  // for a real 2 nb-column unit, one panel for nb columns or fewer, else the
+  // for up to 2 nb real columns, one panel for nb columns or fewer, else the
   // first part, its reflectors applied to the rest's columns, the rest, and
   // the two compact-WY forms merged,
   //   V = [V1 | (0; V2)],  T = [T1, -T1 (V1^H V2) T2; 0, T2].
@@ -744,12 +750,15 @@ int geqrf_dev(Handle* h, int m, int n, T* A, long lda, T* tau, T* B, int nrhs, l
     if constexpr (!S<T>::cplx) {
       // every workgroup of the block kernel must have a CU of the panel set
       const int bcap = std::min(256, h->panel_cap > 0 ? h->panel_cap : h->num_cus);
-      const int Gb = (use_block && w == 2 * nb) ? cqr_block_groups(m - i, bcap) : 0;
+      const int Gb = use_block ? cqr_block_groups(m - i, w, bcap) : 0;
       if (Gb > 0) {
-        // Both panels, the apply between them and the merge in one launch.
         const int p1 = i / nb;
         CqrBlockArgs ba;
         ba.mp = m - i;
+        ba.w = w;
+        // Short and ragged blocks (small matrices, factorizations' ends) keep
+        // the reference's tau = 0 for zero tails; full ones, as ever, tau = 2.
+        ba.zero_tails = w < 2 * nb || m - i < 3 * nb;
         ba.A = A + (size_t)i + (size_t)i * lda;
         ba.lda = lda;
         ba.tau = tau + i;
@@ -914,8 +923,10 @@ int geqrf_dev(Handle* h, int m, int n, T* A, long lda, T* tau, T* B, int nrhs, l
         // there block b+1's kernel can queue behind other requests' work and
         // the gate would hold this stream for nothing.
         const int Gb =
-            use_block ? cqr_block_groups(m - c0, std::min(256, h->panel_cap > 0 ? h->panel_cap : h->num_cus)) : 0;
-        if (wn >= 2 * nb && Gb > 0 && m - c0 <= gate_rows && c0 + wn < n && !h->ext_pstream)
+            use_block ? cqr_block_groups(m - c0, std::min(wn, 2 * nb),
+                                         std::min(256, h->panel_cap > 0 ? h->panel_cap : h->num_cus))
+                      : 0;
+        if (Gb > 0 && m - c0 <= gate_rows && c0 + wn < n && !h->ext_pstream)
           RNPX_TRY(launch_cqr_gate((const unsigned*)h->sync.p + 1 + 2 * npan + (size_t)kCqrSyncWords * (c0 / nb), Gb,
                                    (unsigned*)h->flag.p + kGateOffWord, us));
       }

@@ -8,7 +8,10 @@
 // and the blocks right of it at once; the trailing updates and the inverses'
 // off-diagonal blocks are 16x16x16 block products on FP64 MFMA spread over
 // the four waves, and the diagonal blocks' inverses run on an idle wave
-// beside the next chain.
+// beside the next chain.  The loops over blocks stay rolled and each chain has one
+// copy per caller: everything here runs once or twice per launch, so code that
+// the instruction cache (64 KB, shared by two CUs) has not seen is a large part
+// of its time (unrolled over blocks, the outer-block kernel was 370 KB).
 #pragma once
 #include "rnpx_kernels.hpp"
 
@@ -119,11 +122,12 @@ __device__ __forceinline__ void inv_unit_lower16(const double* M, int b, double*
 template <int S>
 __device__ __forceinline__ void inv_upper_offdiag(const double* M, double* X, double* tmp, int lane, int wave) {
   double* t = tmp + wave * 16 * TS;
-#pragma unroll
+#pragma unroll 1
   for (int d = 1; d < 4; ++d) {
     if (wave < 4 - d) {
       const int i = wave, j = wave + d;
       f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
       for (int k = i + 1; k <= j; ++k) mma16<S, S>(acc, M, i, k, false, X, k, j, false, false, lane);
       store_blk<TS>(acc, t, 0, 0, 1.0, lane);
       f64x4 x = {0.0, 0.0, 0.0, 0.0};
@@ -140,11 +144,12 @@ __device__ __forceinline__ void inv_upper_offdiag(const double* M, double* X, do
 template <int S>
 __device__ __forceinline__ void inv_lower_offdiag(const double* M, double* Z, double* tmp, int lane, int wave) {
   double* t = tmp + wave * 16 * TS;
-#pragma unroll
+#pragma unroll 1
   for (int d = 1; d < 4; ++d) {
     if (wave < 4 - d) {
       const int j = wave, i = wave + d;
       f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
       for (int k = j; k < i; ++k) mma16<S, S>(acc, M, i, k, false, Z, k, j, false, false, lane);
       store_blk<TS>(acc, t, 0, 0, 1.0, lane);
       f64x4 z = {0.0, 0.0, 0.0, 0.0};
@@ -189,9 +194,8 @@ __device__ __forceinline__ bool chol_strip(double* M, int b, const double* gdiag
 // is positive and +1 otherwise (into dsg), at diagonal block b over its
 // block row (ROW: one column per lane; U_bb, L_bb and U_bc for c > b) or its
 // block column (one row per lane; L_cb for c > b).  Both chains apply the
-// same operations to the diagonal block in the same order (l = w inv, then
-// fma(-l, u, w)), so they agree on it bit for bit, pivot signs included;
-// the row chain stores it.  w holds what lu_strip_load read; the two loads
+// same operations to the diagonal block in the same order, so they agree on it
+// bit for bit, pivot signs included; the row chain stores it.  w holds what lu_strip_load read; the two loads
 // must both precede either chain's stores.
 template <int S, bool ROW>
 __device__ __forceinline__ void lu_strip_load(const double* M, int b, double (&w)[16], int lane) {
@@ -200,65 +204,74 @@ __device__ __forceinline__ void lu_strip_load(const double* M, int b, double (&w
   for (int i = 0; i < 16; ++i) w[i] = ROW ? M[(x0 + i) * S + x] : M[x * S + x0 + i];
 }
 template <int S, bool ROW>
-__device__ __forceinline__ void lu_strip(double* M, int b, double (&w)[16], double* dsg, int lane) {
+__device__ __forceinline__ bool lu_strip(double* M, int b, double (&w)[16], double* dsg, int lane, int last,
+                                         double pmax) {
   const int x = lane, x0 = 16 * b;
+  bool ok = true;
+  double mine = 1.0;  // 1 / U(x, x), the scale of this lane's L entries
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
     const int pj = x0 + j;
     const double p = readlane_t(w[j], pj);
-    const double dj = (p > 0.0) ? -1.0 : 1.0;
-    const double u = p - dj;  // |u| = |p| + 1 >= 1
+    const bool none = pj == last;  // no reflector: D takes the pivot's sign, U's entry is a placeholder
+    ok = ok && (none || fabs(p) <= pmax);
+    const double dj = ((p > 0.0) != none) ? -1.0 : 1.0;
+    const double u = none ? 1.0 : p - dj;  // |u| = |p| + 1 >= 1
     const double inv = rcp_nr(u);
+    // element (i, x) -= element(i, pj) * (element(pj, x) inv), element(i, pj) not
+    // yet scaled: the same product in both chains
     if (ROW) {
-      if (x == pj) w[j] = u;
+      const double f = (x > pj) ? -(w[j] * inv) : 0.0;
+      if (x == pj) {
+        w[j] = u;
+        mine = inv;
+      }
       if (lane == 0) dsg[pj] = dj;
 #pragma unroll
-      for (int i = j + 1; i < 16; ++i) {
-        const double lij = readlane_t(w[i], pj) * inv;
-        w[i] = (x > pj) ? fma(-lij, w[j], w[i]) : ((x == pj) ? lij : w[i]);
-      }
+      for (int i = j + 1; i < 16; ++i) w[i] = fma(readlane_t(w[i], pj), f, w[i]);
     } else {
-      const double l = w[j] * inv;
+      const double l = (x > pj) ? w[j] : 0.0;
 #pragma unroll
-      for (int jp = j + 1; jp < 16; ++jp) {
-        const double ujp = readlane_t(w[jp], pj);  // row pj is not updated at step j
-        w[jp] = (x > pj) ? fma(-l, ujp, w[jp]) : w[jp];
-      }
-      w[j] = (x > pj) ? l : ((x == pj) ? u : w[j]);
+      for (int jp = j + 1; jp < 16; ++jp) w[jp] = fma(l, -(readlane_t(w[jp], pj) * inv), w[jp]);
+      w[j] *= inv;
     }
   }
   if (ROW) {
     if (x >= x0) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) M[(x0 + i) * S + x] = w[i];
+      for (int i = 0; i < 16; ++i) M[(x0 + i) * S + x] = (i > x - x0) ? w[i] * mine : w[i];
     }
   } else if (x >= x0 + 16) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) M[x * S + x0 + i] = w[i];
   }
+  return ok;
 }
 
 // All waves: Cholesky M = R^T R of the symmetric 64x64 M in place (R upper;
 // blocks below the diagonal left as they are) and X = R^-1 (upper blocks).
 // Wave 0 runs the block-row chain b while wave 1 inverts diagonal block
-// b-1; all waves share the trailing updates.  Returns the acceptance test
-// (the same in every thread).
+// b-1; all waves share the trailing updates.  gdiag: the squared norms that the
+// acceptance test holds the pivots against (M's own diagonal, or that of the
+// matrix M was updated from), set by the caller.  Returns the test (the same in
+// every thread).
 template <int S>
 __device__ __forceinline__ bool chol64(double* M, double* X, double* tmp, double* gdiag, int* okf, int tid) {
   const int lane = tid & 63, wave = tid >> 6;
   double* rv = tmp + 4 * 16 * TS;  // 4 x 16 reciprocals
-  if (tid < 64) gdiag[tid] = M[tid * S + tid];
   if (tid == 0) *okf = 1;
   __syncthreads();
   bool ok = true;
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    if (wave == 0) ok = chol_strip<S>(M, b, gdiag, lane) && ok;
+#pragma unroll 1
+  for (int b = 0; b < 5; ++b) {
+    if (wave == 0 && b < 4) ok = chol_strip<S>(M, b, gdiag, lane) && ok;
+    if (wave == 0 && b == 4 && lane == 0 && !ok) *okf = 0;
     if (wave == 1 && b > 0) inv_upper16<S, S>(M, b - 1, X, b - 1, rv + 16 * (b - 1), lane);
     __syncthreads();
     if (b < 3) {
       // G_cd -= R_bc^T R_bd for b < c <= d
       const int n = 3 - b, npairs = n * (n + 1) / 2;
+#pragma unroll 1
       for (int e = wave; e < npairs; e += 4) {
         int c = 0, rem = e;
         while (rem >= n - c) {
@@ -274,35 +287,39 @@ __device__ __forceinline__ bool chol64(double* M, double* X, double* tmp, double
       __syncthreads();
     }
   }
-  if (wave == 1) inv_upper16<S, S>(M, 3, X, 3, rv + 48, lane);
-  if (wave == 0 && lane == 0 && !ok) *okf = 0;
-  __syncthreads();
   inv_upper_offdiag<S>(M, X, tmp, lane, wave);  // ends with a barrier
   return *okf != 0;
 }
 
 // All waves: M (64x64, holding Q_top) := the LU factors of M - D (U on and
 // above the diagonal, unit lower L below), D into dsg, X = U^-1 (upper
-// blocks).  The block-row and block-column chains of step b run side by
+// blocks).  Column `last` (-1: none), the last of a square matrix, has no
+// reflector.  Returns whether every other running pivot is at most pmax in
+// magnitude (the same in every thread).  The block-row and block-column chains of step b run side by
 // side on waves 0 and 1 while wave 2 inverts U's diagonal block b-1.
 template <int S>
-__device__ __forceinline__ void lu64(double* M, double* dsg, double* X, double* tmp, int tid) {
+__device__ __forceinline__ bool lu64(double* M, double* dsg, double* X, double* tmp, int* okf, int tid, int last = -1,
+                                     double pmax = 2.0) {
   const int lane = tid & 63, wave = tid >> 6;
+  if (tid == 0) *okf = 1;
+  bool ok = true;
   double* rv = tmp + 4 * 16 * TS;  // 4 x 16 reciprocals
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
+#pragma unroll 1
+  for (int b = 0; b < 5; ++b) {
     double w[16];
     // the column chain reads the diagonal block the row chain overwrites
-    if (wave == 0) lu_strip_load<S, true>(M, b, w, lane);
+    if (wave == 0 && b < 4) lu_strip_load<S, true>(M, b, w, lane);
     if (wave == 1 && b < 3) lu_strip_load<S, false>(M, b, w, lane);
     if (b < 3) __syncthreads();
-    if (wave == 0) lu_strip<S, true>(M, b, w, dsg, lane);
-    if (wave == 1 && b < 3) lu_strip<S, false>(M, b, w, dsg, lane);
+    if (wave == 0 && b == 4 && lane == 0 && !ok) *okf = 0;
+    if (wave == 0 && b < 4) ok = lu_strip<S, true>(M, b, w, dsg, lane, last, pmax) && ok;
+    if (wave == 1 && b < 3) (void)lu_strip<S, false>(M, b, w, dsg, lane, last, pmax);
     if (wave == 2 && b > 0) inv_upper16<S, S>(M, b - 1, X, b - 1, rv + 16 * (b - 1), lane);
     __syncthreads();
     if (b < 3) {
       // W_cd -= L_cb U_bd for c, d > b
       const int n = 3 - b;
+#pragma unroll 1
       for (int e = wave; e < n * n; e += 4) {
         const int c = b + 1 + e / n, d = b + 1 + e % n;
         f64x4 acc;
@@ -313,9 +330,8 @@ __device__ __forceinline__ void lu64(double* M, double* dsg, double* X, double* 
       __syncthreads();
     }
   }
-  if (wave == 2) inv_upper16<S, S>(M, 3, X, 3, rv + 48, lane);
-  __syncthreads();
-  inv_upper_offdiag<S>(M, X, tmp, lane, wave);
+  inv_upper_offdiag<S>(M, X, tmp, lane, wave);  // ends with a barrier
+  return *okf != 0;
 }
 
 // All waves: Z = L^-1 for the unit lower triangle below the diagonal of M.
