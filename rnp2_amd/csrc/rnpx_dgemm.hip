@@ -152,6 +152,7 @@ struct Args {
   int kslice;  // K per split slice (multiple of BK)
   int tilesM, tilesN, ntiles;
   long sa, sb, sc;  // strided batch (grid y): elements between the problems' A, B, C
+  int mlast;        // batched Grams: M and N of the last problem (0: as the others)
 };
 
 // Workgroup -> (tile m, tile n, split z): contiguous chunks per XCD, then
@@ -229,6 +230,7 @@ __global__ __launch_bounds__(kThreads) void dgemm_kernel(Args a0) {
   a.A += (size_t)blockIdx.y * a0.sa;
   a.B += (size_t)blockIdx.y * a0.sb;
   a.C += (size_t)blockIdx.y * a0.sc;
+  if (a0.mlast && blockIdx.y == gridDim.y - 1) a.M = a.N = a0.mlast;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
@@ -659,13 +661,14 @@ hipError_t dgemm_mfma_batched(int M, int N, int K, double alpha, const double* A
   }
 }
 
-// Grams of consecutive column blocks of V in one launch: block b (w columns at
-// V + b w ldv, n rows) split over the rows into ns slices of kslice, the raw
-// slices at part + (b ns + z) ldp^2 (w x w, leading dimension ldp).  64 x 64
+// Grams of consecutive column blocks of V in one launch: block b (w columns,
+// the last one wlast, at V + b w ldv, n rows) split over the rows into ns slices of
+// kslice, the raw slices at part + (b ns + z) w^2.  64 x 64
 // tiles: the blocks are few and the slices are what fills the chip.
-hipError_t dgemm_gram_batched(int n, int w, int ldp, const double* V, long ldv, int kslice, int ns, double* part,
+hipError_t dgemm_gram_batched(int n, int w, int wlast, const double* V, long ldv, int kslice, int ns, double* part,
                               int batch, hipStream_t st) {
-  if (n < 1 || w < 1 || ldp < w || ldv < n || batch < 1 || batch > 65535 || ns < 1 || kslice < 16 || kslice % 16)
+  if (n < 1 || w < 1 || wlast < 1 || wlast > w || ldv < n || batch < 1 || batch > 65535 || ns < 1 || kslice < 16 ||
+      kslice % 16)
     return hipErrorInvalidValue;
   dg::Args a{};
   a.M = a.N = w;
@@ -677,9 +680,10 @@ hipError_t dgemm_gram_batched(int n, int w, int ldp, const double* V, long ldv, 
   a.mode = dg::kSplit;
   a.kslice = kslice;
   a.C = part;
-  a.ldc = ldp;
-  a.zstride = (size_t)ldp * ldp;
-  a.sc = (long)ldp * ldp * ns;
+  a.ldc = w;
+  a.zstride = (size_t)w * w;
+  a.sc = (long)w * w * ns;
+  a.mlast = wlast;
   return dg::launch<true, true, 64, 64, 16>(a, st, batch);
 }
 

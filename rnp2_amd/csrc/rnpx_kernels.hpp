@@ -105,19 +105,19 @@ __device__ __forceinline__ void wait_flag(unsigned* flag, unsigned* abortf) {
 }
 
 // Sum of p[q * stride] over q < n, added in the order of q (the result is
-// that of the plain loop), with eight loads in flight instead of one.
+// that of the plain loop), with sixteen loads in flight instead of one (a last,
+// shorter batch reads its end again instead of going one by one).
 template <typename T>
 __device__ __forceinline__ T sum_strided(const T* p, int n, size_t stride) {
   T s = S<T>::zero();
-  int q = 0;
-  for (; q + 8 <= n; q += 8) {
-    T v[8];
+  for (int q = 0; q < n; q += 16) {
+    T v[16];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = p[(size_t)(q + u) * stride];
+    for (int u = 0; u < 16; ++u) v[u] = p[(size_t)min(q + u, n - 1) * stride];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) s = s + v[u];
+    for (int u = 0; u < 16; ++u)
+      if (q + u < n) s = s + v[u];
   }
-  for (; q < n; ++q) s = s + p[(size_t)q * stride];
   return s;
 }
 
@@ -301,9 +301,9 @@ hipError_t launch_gram_blocks(int n, int k, int w, const T* V, long ldv, const T
                               hipStream_t st);
 template <typename T>
 hipError_t launch_tfactor_blocks(const T* gram, int w, int k, T* Tout, hipStream_t st);
-hipError_t dgemm_gram_batched(int n, int w, int ldp, const double* V, long ldv, int kslice, int ns, double* part,
+hipError_t dgemm_gram_batched(int n, int w, int wlast, const double* V, long ldv, int kslice, int ns, double* part,
                               int batch, hipStream_t st);
-hipError_t zgemm_gram_batched(int n, int w, int ldp, const zd* V, long ldv, int kslice, int ns, zd* part, int batch,
+hipError_t zgemm_gram_batched(int n, int w, int wlast, const zd* V, long ldv, int kslice, int ns, zd* part, int batch,
                               hipStream_t st);
 
 // General matrix multiply on FP64 MFMA:

@@ -332,11 +332,11 @@ static int pick_ksplit(const Handle* h, int rows, int cols_tiles) {
   // tuning says.
   if (h->tune.ksplit > 0 && cols_tiles > 2) return h->tune.ksplit;
   // About 512 workgroup tiles of 128 x 128 in all (two per CU; measured best
-  // for W = V^H C at 4096-8192 rows).  K slices of at least 512, or 128 for
+  // for W = V^H C at 4096-8192 rows).  K slices of at least 512, or 64 for
   // the narrow products (one or two column tiles) that sit on the chain of
   // panels, where latency matters more than the partial sums' traffic.
   int want = (cols_tiles <= 2 ? 1024 : 512) / std::max(1, cols_tiles);
-  int maxs = std::max(1, rows / (cols_tiles <= 2 ? 128 : 512));
+  int maxs = std::max(1, rows / (cols_tiles <= 2 ? 64 : 512));
   // narrow products: up to 64 slices (a tall panel's W is otherwise a long
   // chain of K slices on few workgroups)
   return std::max(1, std::min(want, std::min(maxs, cols_tiles <= 2 ? 64 : 32)));
@@ -465,7 +465,9 @@ struct WyPlan {
 // 2.21 ms, GenerateQ of 8192 x 2048 from 5.77 to 2.31 ms.
 template <typename T>
 static int wy_plan(Handle* h, bool own_v, bool left, int nq, int k, int rows, int cols, bool shrink, WyPlan* out) {
-  const int wide = S<T>::cplx ? 64 : (k > 64 ? 128 : 64), narrow = S<T>::cplx ? 32 : 64;
+  // no wider than the reflectors: a T leaf of 64 complex columns takes 30 us where
+  // one of 32 takes 15
+  const int wide = S<T>::cplx ? (k > 32 ? 64 : 32) : (k > 64 ? 128 : 64), narrow = S<T>::cplx ? 32 : 64;
   const int most = own_v ? std::min(k, 2048) : k;
   const WyPlan tries[3] = {{wide, (most + wide - 1) / wide * wide}, {wide, wide}, {narrow, narrow}};
   for (int t = h->budget ? 2 : 0; t < 3; ++t) {
@@ -473,7 +475,7 @@ static int wy_plan(Handle* h, bool own_v, bool left, int nq, int k, int rows, in
     const int cw = std::min(p.chunk, k), nblk = (cw + p.w - 1) / p.w;
     const size_t ws = sizeof(T) * (size_t)p.w * p.w;
     // slices of the Grams, of this chunk or a shorter last one
-    const int per = std::min(64, std::max(1, nq / 256));
+    const int per = std::min(96, std::max(1, nq / 32));
     const size_t nsl = std::min(per * nblk, std::max(nblk, 768 / (p.w <= 64 ? 1 : 4)));
     size_t wz = 0, part = 0;
     for (int i = 0; i < k; i += p.w) {

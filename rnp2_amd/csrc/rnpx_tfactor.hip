@@ -144,8 +144,10 @@ __global__ void gram_sum_blocks_kernel(int k, int w, int ns, const T* __restrict
 
 int gram_blocks_slices(int n, int k, int w, int* kslice) {
   const int nblk = (k + w - 1) / w, tiles = (w <= 64 ? 1 : 4) * nblk;
-  // about three workgroups per CU in all, slices of at least 256 rows
-  int ns = std::max(1, std::min({64, n / 256, 768 / tiles}));
+  // about three workgroups per CU in all, slices of at least 32 rows (16 rows
+  // of a slice take about a microsecond, whatever else is idle) and at most
+  // 96 of them (their sum takes about half a microsecond for eight)
+  int ns = std::max(1, std::min({96, n / 32, 768 / tiles}));
   *kslice = ((n + ns - 1) / ns + 15) / 16 * 16;
   return (n + *kslice - 1) / *kslice;
 }
@@ -157,17 +159,12 @@ hipError_t launch_gram_blocks(int n, int k, int w, const T* V, long ldv, const T
   int kslice = 0;
   const int ns = gram_blocks_slices(n, k, w, &kslice), full = k / w, rest = k - full * w;
   const size_t ws = (size_t)w * w;
-  for (int r = 0; r < 2; ++r) {  // the full blocks, then a narrower last one
-    const int nb = r == 0 ? full : (rest > 0), cols = r == 0 ? w : rest;
-    if (nb == 0) continue;
-    const T* Vr = V + (r == 0 ? 0 : (size_t)full * w * ldv);
-    T* pr = part + (r == 0 ? 0 : full * ns * ws);
-    if constexpr (S<T>::cplx)
-      RNPX_LAUNCH_CHECK(zgemm_gram_batched(n, cols, w, Vr, ldv, kslice, ns, pr, nb, st));
-    else
-      RNPX_LAUNCH_CHECK(dgemm_gram_batched(n, cols, w, Vr, ldv, kslice, ns, pr, nb, st));
-  }
-  hipLaunchKernelGGL((gram_sum_blocks_kernel<T>), dim3((unsigned)((ws + 255) / 256), full + (rest > 0)), dim3(256), 0,
+  const int nblk = full + (rest > 0), wlast = rest > 0 ? rest : w;
+  if constexpr (S<T>::cplx)
+    RNPX_LAUNCH_CHECK(zgemm_gram_batched(n, w, wlast, V, ldv, kslice, ns, part, nblk, st));
+  else
+    RNPX_LAUNCH_CHECK(dgemm_gram_batched(n, w, wlast, V, ldv, kslice, ns, part, nblk, st));
+  hipLaunchKernelGGL((gram_sum_blocks_kernel<T>), dim3((unsigned)((ws + 255) / 256), nblk), dim3(256), 0,
                      st, k, w, ns, part, tau, gram);
   return hipGetLastError();
 }

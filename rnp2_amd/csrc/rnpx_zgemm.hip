@@ -104,6 +104,7 @@ struct Args {
   int tilesM, tilesN;
   int conja;  // op(A) = 'C'
   long sa, sb, sc;  // strided batch (grid y): elements between the problems' A, B, C
+  int mlast;        // batched Grams: M and N of the last problem (0: as the others)
 };
 
 // Workgroup -> (tile m, tile n, split z): contiguous chunks per XCD, then
@@ -135,6 +136,7 @@ __global__ __launch_bounds__(kThreads) void zgemm_kernel(Args a0) {
   a.A += (size_t)blockIdx.y * a0.sa;
   a.B += (size_t)blockIdx.y * a0.sb;
   a.C += (size_t)blockIdx.y * a0.sc;
+  if (a0.mlast && blockIdx.y == gridDim.y - 1) a.M = a.N = a0.mlast;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
@@ -307,9 +309,10 @@ hipError_t zgemm_mfma(char ta, char tb, int M, int N, int K, zd alpha, const zd*
 }
 
 // Batched Grams V_b^H V_b, as dgemm_gram_batched.
-hipError_t zgemm_gram_batched(int n, int w, int ldp, const zd* V, long ldv, int kslice, int ns, zd* part, int batch,
+hipError_t zgemm_gram_batched(int n, int w, int wlast, const zd* V, long ldv, int kslice, int ns, zd* part, int batch,
                               hipStream_t st) {
-  if (n < 1 || w < 1 || ldp < w || ldv < n || batch < 1 || batch > 65535 || ns < 1 || kslice < 16 || kslice % 16)
+  if (n < 1 || w < 1 || wlast < 1 || wlast > w || ldv < n || batch < 1 || batch > 65535 || ns < 1 || kslice < 16 ||
+      kslice % 16)
     return hipErrorInvalidValue;
   zg::Args a{};
   a.M = a.N = w;
@@ -322,9 +325,11 @@ hipError_t zgemm_gram_batched(int n, int w, int ldp, const zd* V, long ldv, int 
   a.mode = zg::kSplit;
   a.kslice = kslice;
   a.C = part;
-  a.ldc = ldp;
-  a.zstride = (size_t)ldp * ldp;
-  a.sc = (long)ldp * ldp * ns;
+  a.ldc = w;
+  a.zstride = (size_t)w * w;
+  a.sc = (long)w * w * ns;
+  a.mlast = wlast;
+  if (w <= 32) return zg::launch<true, 32, 64, 16>(a, ns, st, batch);
   return zg::launch<true, 64, 64, 16>(a, ns, st, batch);
 }
 
