@@ -587,9 +587,10 @@ static int panel_step(Handle* h, int p, int npan, int i, int ib, int m, int nb, 
 
 // Factor (QR.hpp:129-197) on device memory.
 //
-// Outer blocks of nbo = 2 nb columns (the default; nb = 64) are factored as
-// two inner panels of nb columns: panel 1, its block reflector applied to
-// the next nb columns, panel 2, then the two compact-WY forms are merged,
+// Outer blocks of nbo = 2 nb columns (the default; nb = 64) are one launch of the
+// outer-block kernel (real, use_block), else two inner panels of nb columns:
+// panel 1, its block reflector applied to the next nb columns, panel 2, then the
+// two compact-WY forms are merged,
 //   V = [V1 | (0; V2)],  T = [T1, -T1 (V1^H V2) T2; 0, T2],
 // so that the trailing matrix sees one rank-nbo update (K = 128 GEMMs run
 // half as many passes over it at higher arithmetic intensity than K = 64).

@@ -68,9 +68,10 @@ static double now_s() {
 // to the server's list when a request is done, so that a submit neither faults
 // fresh pages in nor clears them before the copy (submitting a burst of 24
 // requests, 340 MB, took 63 ms that way and takes 9 now; the burst 74.5 -> 45.2
-// ms), and the worker's transfer to the device is one asynchronous DMA.  At most kPinnedBytes in all, in use or idle,
-// given back when the server is destroyed; a request beyond that (or where
-// pinned memory is refused) takes ordinary memory.
+// ms), and the worker's transfer to the device is one asynchronous DMA.  At
+// most kPinnedBytes in all, in use or idle, given back when the server is
+// destroyed; a request beyond that (or where pinned memory is refused) takes
+// ordinary memory.
 struct HostBlock {
   double* p = nullptr;
   size_t bytes = 0;

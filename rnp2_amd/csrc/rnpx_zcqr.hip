@@ -35,13 +35,12 @@ namespace rnpx {
 
 namespace zq {
 
-// The small products and the second pass's exact factorization: one workgroup of
-// LPC lanes per column; thread t
-// holds rows (t mod LPC) + LPC r (r < NB / LPC) of column t / LPC of the
-// 32 x 32 matrix being worked on in registers, so the lanes of a column sit
-// in one wave and share values by shuffles; a matrix other columns read is
-// staged in LDS.  A Cholesky or LU step costs one workgroup barrier, a
-// triangular inverse or product none.
+// The small products, R's and U's inverses and the second pass's exact Cholesky:
+// one workgroup of LPC lanes per column; thread t holds rows
+// (t mod LPC) + LPC r (r < NB / LPC) of column t / LPC of the 32 x 32 matrix being
+// worked on in registers, so the lanes of a column sit in one wave and share
+// values by shuffles; a matrix other columns read is staged in LDS.  A step of
+// that Cholesky costs one workgroup barrier, a triangular inverse or product none.
 constexpr int NB = 32;
 constexpr int LPC = 8;  // lanes per column (measured: 4 and 16 are slower)
 constexpr int kSmall = NB * LPC;
