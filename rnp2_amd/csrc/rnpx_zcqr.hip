@@ -35,12 +35,12 @@ namespace rnpx {
 
 namespace zq {
 
-// The small products, R's and U's inverses and the second pass's exact Cholesky:
-// one workgroup of LPC lanes per column; thread t holds rows
+// The reconstruction (and the second pass's exact Cholesky): one workgroup of LPC
+// lanes per column; thread t holds rows
 // (t mod LPC) + LPC r (r < NB / LPC) of column t / LPC of the 32 x 32 matrix being
 // worked on in registers, so the lanes of a column sit in one wave and share
-// values by shuffles; a matrix other columns read is staged in LDS.  A step of
-// that Cholesky costs one workgroup barrier, a triangular inverse or product none.
+// values by shuffles; a matrix other columns read is staged in LDS.  A Cholesky
+// or LU step costs one workgroup barrier, a triangular inverse or product none.
 constexpr int NB = 32;
 constexpr int LPC = 8;  // lanes per column (measured: 4 and 16 are slower)
 constexpr int kSmall = NB * LPC;
@@ -109,13 +109,17 @@ __device__ __forceinline__ bool chol_cols(zd (&g)[R4], int c, int sub, double re
 
 // Column c of X = U^{-1} for the upper triangular U in LDS (entries below
 // its diagonal never read), by the column sweep y = e_c, x_k = y_k / U_kk,
-// y_i -= U_ik x_k (i < k), k = NB-1 .. 0.
+// y_i -= U_ik x_k (i < k), k = NB-1 .. 0.  unit: U_kk = 1.  conjT: U_ik is
+// conj(L(k, i)) of the lower triangular L stored there instead.
 // The reciprocals of U's diagonal are formed first, in parallel, into rdiag
 // (LDS), off the sweep's serial chain.  Whole workgroup.
+template <bool UNIT, bool CONJT>
 __device__ __forceinline__ void inv_upper_col(const Mat& U, int c, int sub, zd (&x)[R4], zd* rdiag) {
-  __syncthreads();  // earlier readers of rdiag are done
-  if (threadIdx.x < NB) rdiag[threadIdx.x] = zrecip(U[threadIdx.x][threadIdx.x]);
-  __syncthreads();
+  if constexpr (!UNIT) {
+    __syncthreads();  // earlier readers of rdiag are done
+    if (threadIdx.x < NB) rdiag[threadIdx.x] = zrecip(U[threadIdx.x][threadIdx.x]);
+    __syncthreads();
+  }
 #pragma unroll
   for (int r = 0; r < R4; ++r) x[r] = (sub + LPC * r == c) ? S<zd>::one() : S<zd>::zero();
   // k = LPC rk + s: rk unrolled (a fixed register), s not
@@ -124,14 +128,16 @@ __device__ __forceinline__ void inv_upper_col(const Mat& U, int c, int sub, zd (
 #pragma unroll 1
     for (int s8 = LPC - 1; s8 >= 0; --s8) {
       const int k = LPC * rk + s8;
-      const zd xk = gbcast(x[rk] * rdiag[k], s8);
+      zd xk = x[rk];
+      if constexpr (!UNIT) xk = xk * rdiag[k];
+      xk = gbcast(xk, s8);
 #pragma unroll
       for (int r = 0; r < R4; ++r) {
         const int i = sub + LPC * r;
         if (i == k)
           x[r] = xk;
         else if (i < k)
-          x[r] = x[r] - U[i][k] * xk;
+          x[r] = x[r] - (CONJT ? zconj(U[k][i]) : U[i][k]) * xk;
       }
     }
   }
@@ -157,7 +163,7 @@ __device__ __forceinline__ void mul_col(const Mat& A, const zd (&b)[R4], int sub
   }
 }
 
-// ---- 32 x 32 factorizations on one wave ----
+// ---- the first pass's 32 x 32 Cholesky on one wave ----
 // Lane c < 32 holds column c of the matrix, lane 32 + c column c of the identity,
 // all rows in registers: the elimination's row operations on [G | I] leave the
 // triangular factor in the left lanes and the inverse of the eliminated one in the
@@ -210,51 +216,12 @@ __device__ __forceinline__ bool chol_wave(ZCol& a, double dg, double rel) {
   return ok;
 }
 
-// LU without pivoting of [Q - D | I], D_j = -sign(Re pivot) (+1 for a zero real
-// part): U (left lanes, rows <= c), the unit lower L (left lanes, rows > c) and
-// L^{-1} (right lanes); dsg: D_c in lane c.
-__device__ __forceinline__ void lu_wave(ZCol& a, double& dsg, int lane) {
-  zd mine = S<zd>::one();  // 1 / U(c, c), the scale of this lane's L entries
-#pragma unroll 1
-  for (int b = 0; b < NB / 4; ++b) {
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const int j = 4 * b + s;
-      const zd p = readlane_t(a.w[s], j);
-      const double dj = p.x > 0.0 ? -1.0 : 1.0;
-      const zd u = mkz(p.x - dj, p.y);  // |u| >= 1: no scaling in its reciprocal
-      const double n2 = small64::rcp_nr(fma(u.x, u.x, u.y * u.y));
-      const zd inv = mkz(u.x * n2, -u.y * n2);
-      const zd f = sel(lane > j, S<zd>::zero() - a.w[s] * inv, S<zd>::zero());
-      if (lane == j) {
-        a.w[s] = u;
-        mine = inv;
-        dsg = dj;
-      }
-#pragma unroll
-      for (int q = 0; q < NB / 4; ++q)
-        if (q < NB / 4 - b) {
-#pragma unroll
-          for (int i = 4 * q; i < 4 * q + 4; ++i)
-            if (i > s) {
-              const zd l = readlane_t(a.w[i], j);  // L(row of i, j) U(j, j)
-              a.w[i].x = fma(-l.y, f.y, fma(l.x, f.x, a.w[i].x));
-              a.w[i].y = fma(l.y, f.x, fma(l.x, f.y, a.w[i].y));
-            }
-        }
-    }
-    rotate4(a);
-  }
-  if (lane < NB) {
-#pragma unroll
-    for (int i = 0; i < NB; ++i) a.w[i] = sel(i > lane, a.w[i] * mine, a.w[i]);
-  }
-}
-
 // Pass 1: R1 = chol(G1) and R1^{-1}, or the fail flag; one wave, since the kernel
 // is one serial chain: 25 us, 32 with a barrier, a square root and a division per
 // step over four waves and a substitution for the inverse.  0.6 us a step, the
-// row updates' v_readlanes and the branches between them.
+// row updates' v_readlanes and the branches between them.  (The reconstruction's
+// LU the same way took that kernel from 44 to 46 us: its steps already overlapped
+// the division with the row updates, which one wave does alone.)
 __global__ __launch_bounds__(64) void chol_kernel(const zd* __restrict__ G, zd* __restrict__ R1,
                                                   zd* __restrict__ R1i, unsigned* fail) {
   const int lane = threadIdx.x, c = lane & 31;
@@ -347,7 +314,7 @@ __global__ __launch_bounds__(kSmall) void recon_kernel(const zd* __restrict__ G2
       return;
     }
     to_lds(S1, c, sub, g);  // R2
-    inv_upper_col(S1, c, sub, x2, rowb[0]);  // column c of R2^{-1}
+    inv_upper_col<false, false>(S1, c, sub, x2, rowb[0]);  // column c of R2^{-1}
   }
   if (!ok) {
     if (t == 0) *fail = 1u;
@@ -358,24 +325,42 @@ __global__ __launch_bounds__(kSmall) void recon_kernel(const zd* __restrict__ G2
   // q = column c of Q_top = Q1_top R2^{-1}
   zd q[R4];
   mul_col(S3, x2, sub, q);
-  // LU without pivoting of Q_top - D: L1 strictly below, U on and above, and
-  // L1^{-1}, by one wave; S3 (Q1's top) is done with
-  to_lds(S4, c, sub, q);
-  __syncthreads();
-  if (t < 64) {
-    const int cc = t & 31;
-    ZCol a;
-    double dsg = 1.0;
+  // LU without pivoting of Q_top - D: L1 strictly below, U on and above;
+  // D_j = -sign(Re pivot) (+1 for a zero real part)
+  zd (*Lc)[NB] = rowb;
 #pragma unroll
-    for (int i = 0; i < NB; ++i) a.w[i] = t < NB ? S4[i][cc] : (i == cc ? S<zd>::one() : S<zd>::zero());
-    lu_wave(a, dsg, t);
+  for (int rj = 0; rj < R4; ++rj)
+#pragma unroll 1
+  for (int s8 = 0; s8 < LPC; ++s8) {
+    const int j = LPC * rj + s8;
+    if (c == j) {
+      const zd piv = gbcast(q[rj], s8);
+      const double dj = piv.x > 0.0 ? -1.0 : 1.0;
+      const zd pivp = mkz(piv.x - dj, piv.y);
+      const zd rp = zrecip(pivp);
 #pragma unroll
-    for (int i = 0; i < NB; ++i) (t < NB ? S4 : S3)[i][cc] = a.w[i];
-    if (t < NB) Ds[t] = dsg;
+      for (int r = 0; r < R4; ++r) {
+        const int i = sub + LPC * r;
+        if (i == j) {
+          q[r] = pivp;
+        } else if (i > j) {
+          q[r] = q[r] * rp;
+          Lc[j & 1][i] = q[r];
+        }
+      }
+      if (sub == 0) Ds[j] = dj;
+    }
+    __syncthreads();
+    if (c > j) {
+      const zd u = gbcast(q[rj], s8);  // U(j, c)
+#pragma unroll
+      for (int r = 0; r < R4; ++r) {
+        const int i = sub + LPC * r;
+        if (i > j) q[r] = q[r] - Lc[j & 1][i] * u;
+      }
+    }
   }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < R4; ++r) q[r] = S4[sub + LPC * r][c];
+  to_lds(S4, c, sub, q);
   // R = D R2 R1 (upper) and L1 (strictly lower) -> Atop; V's top rows = unit L1
   {
     zd r1[R4], rr[R4];
@@ -393,16 +378,17 @@ __global__ __launch_bounds__(kSmall) void recon_kernel(const zd* __restrict__ G2
   // M = R2^{-1} U^{-1}
   {
     zd ui[R4], mm[R4];
-    inv_upper_col(S4, c, sub, ui, rowb[0]);
+    inv_upper_col<false, false>(S4, c, sub, ui, rowb[0]);
     mul_col(S2, ui, sub, mm);
 #pragma unroll
     for (int r = 0; r < R4; ++r)
       if (sub + LPC * r > c) mm[r] = S<zd>::zero();
     store_col(M, NB, c, sub, mm);
   }
-  // T = -(U D) L1^{-H}
+  // T = -(U D) L1^{-H}: Y = L1^{-H}, the inverse of the unit upper L1^H
   {
-    zd tt[R4];
+    zd y[R4], tt[R4];
+    inv_upper_col<true, true>(S4, c, sub, y, rowb[0]);
     // (U D) with U the upper part of S4: entries below the diagonal masked
     zd u[R4];
 #pragma unroll
@@ -412,7 +398,7 @@ __global__ __launch_bounds__(kSmall) void recon_kernel(const zd* __restrict__ G2
 #pragma unroll 2
     for (int s8 = 0; s8 < LPC; ++s8) {
       const int l = LPC * rl + s8;
-      const zd yl = zconj(S3[c][l]);
+      const zd yl = gbcast(y[rl], s8);
 #pragma unroll
       for (int r = 0; r < R4; ++r) {
         const int i = sub + LPC * r;
