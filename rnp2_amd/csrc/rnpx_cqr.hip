@@ -537,14 +537,11 @@ static_assert(kBlkResident < kCqrBlockSyncWords, "block sync words");
 constexpr int kCross = 16 * 256;                   // a 64x64 product in 16 tiles
 constexpr int kBlkElems = kCqrBlockPart;           // upper tiles of a 128x128 Gram: G11, G12, G22
 static_assert(2 * kGramElems + kCross == kBlkElems, "Gram layout: tiles 0..9, 10..25, 26..35");
-constexpr int kBlkPasses = 3;                      // Cholesky passes at most (and one first-order pass)
+constexpr int kBlkPasses = blk::kPasses;
 constexpr double kThirdPass = 0x1p-3;
 constexpr unsigned kRejected = 2u;                 // flag value: the block goes column by column
-// scratch (doubles): R11, R12, R22 of each pass, then the published blocks;
-// the column-wise refactorization's Gram and T reuse the front
-constexpr int kBR = 0, kBU1i = 3 * 4096 * (kBlkPasses + 1), kBU12 = kBU1i + 4096, kBT1 = kBU12 + 4096,
-              kBU2i = kBT1 + 4096, kBD1 = kBU2i + 4096, kBD2 = kBD1 + 64, kBG = 0, kBTF = 16384;
-static_assert(kBD2 + 64 <= kCqrBlockScratch && kBTF + 16384 <= kCqrBlockScratch, "block scratch");
+constexpr int kBR = blk::kR, kBU1i = blk::kU1i, kBU12 = blk::kU12, kBT1 = blk::kT1, kBU2i = blk::kU2i,
+              kBD1 = blk::kD1, kBD2 = blk::kD2, kBG = blk::kGram, kBTF = blk::kTFactor;
 
 // wait_flag, and the flag's value in every thread.
 __device__ __forceinline__ unsigned wait_verdict(unsigned* flag, unsigned* abortf, unsigned* slot) {

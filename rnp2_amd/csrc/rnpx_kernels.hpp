@@ -3,6 +3,7 @@
 // given against what its kernel and grid assume and returns
 // hipErrorInvalidValue instead of launching when they do not match.
 #pragma once
+#include "rnpx_cqr_layout.hpp"
 #include "rnpx_device.hpp"
 #include "../../include/rnpx.h"
 
@@ -270,7 +271,7 @@ struct CqrBlockArgs {
   unsigned* fail;       // zero at launch; 1 = refactored column by column
 };
 constexpr int kCqrBlockSyncWords = 256;
-constexpr int kCqrBlockScratch = 65728;
+constexpr int kCqrBlockScratch = blk::kScratch;
 constexpr int kCqrBlockPart = 36 * 256;  // the upper 16 x 16 tiles of a 128 x 128 Gram
 // Workgroups for an mp-row, w-column block, 0 when the block kernel does not apply.
 int cqr_block_groups(int mp, int w, int max_groups);
