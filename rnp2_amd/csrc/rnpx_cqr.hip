@@ -499,7 +499,7 @@ __global__ __launch_bounds__(256) void cqr_panel_kernel(CqrArgs a) {
 //      squared norm, a squared norm is outside [2^-600, 2^600] or a value is
 //      not finite.  Every workgroup takes the same decision from the same
 //      reduced Gram, and A is untouched until the block is accepted; a rejected
-//      block is refactored column by column by workgroup 0.
+//      block is refactored column by column (blk_columnwise).
 //   3. Reconstruction [Q1 Q2] - [D; 0] = L U without another reduction:
 //      workgroup 0 factors Q1's top block (L11, U11, D1) and forms
 //      U12 = L11^-1 Q2(0:64), everybody V1 = Q1 U11^-1 and Q2 - V1 U12,
@@ -514,7 +514,8 @@ __global__ __launch_bounds__(256) void cqr_panel_kernel(CqrArgs a) {
 // pivot's own sign and T's column is zero.  Any other column whose entries
 // below the diagonal are exactly zero has no reflector either, which the
 // reconstruction cannot tell from tiny entries (both give tau = 2 to rounding):
-// with zero_tails such a block (a running pivot within 2^-40 of one) is rejected.
+// in the halves named by zero_tails such a running pivot (within 2^-40 of one)
+// rejects the block.
 // Bound by the chain of two grid reductions, two Cholesky and two LU
 // factorizations of 64 x 64.  Against two 64-column panels joined inside the
 // launch (six reductions, the second panel's Gram after the first one's
@@ -541,7 +542,8 @@ constexpr int kBlkPasses = blk::kPasses;
 constexpr double kThirdPass = 0x1p-3;
 constexpr unsigned kRejected = 2u;                 // flag value: the block goes column by column
 constexpr int kBR = blk::kR, kBU1i = blk::kU1i, kBU12 = blk::kU12, kBT1 = blk::kT1, kBU2i = blk::kU2i,
-              kBD1 = blk::kD1, kBD2 = blk::kD2, kBG = blk::kGram, kBTF = blk::kTFactor;
+              kBD1 = blk::kD1, kBD2 = blk::kD2, kBG = blk::kGram, kBTF = blk::kTFactor,
+              kBRow = blk::kRow;
 
 // wait_flag, and the flag's value in every thread.
 __device__ __forceinline__ unsigned wait_verdict(unsigned* flag, unsigned* abortf, unsigned* slot) {
@@ -808,13 +810,12 @@ __device__ __forceinline__ bool one_copy(bool b) {
   return v != 0;
 }
 
-// Rejected block: its w columns column by column in place (team_factor),
-// the clean V, and T from V's Gram by the recursion of
+// Rejected block with norms that need scaling: its w columns column by column in
+// place (team_factor), the clean V, and T from V's Gram by the recursion of
 // GenerateBlockTr("F","C") (Reflector.hpp:580-626), the Gram and T held in
-// scratch.  One workgroup; the others have left.
+// scratch.  One workgroup; no other reads or writes the block any more.
 __device__ __noinline__ void blk_refactor(CqrBlockArgs a, double* sh, int tid) {
   const int K = a.w, mp = a.mp;
-  if (tid == 0) *a.fail = 1u;
   double* Gm = a.scratch + kBG;
   double* Tm = a.scratch + kBTF;
   team_factor<double, 256, true>(mp, K, a.A, (int)a.lda, a.tau, sh);
@@ -847,6 +848,165 @@ __device__ __noinline__ void blk_refactor(CqrBlockArgs a, double* sh, int tid) {
     const int i = e % K, j = e / K;
     a.T[(size_t)i + (size_t)j * a.ldt] = Tm[i * K + j];
   }
+}
+
+typedef __attribute__((address_space(3))) double LdsD;
+
+// Rejected block: column by column by every workgroup, its 64 rows in registers
+// (a thread 32 rows of one column), with Reflector::Generate's rules
+// (Reflector.hpp:117-158).  One grid-wide step per column c: every workgroup
+// hands out its part of x^T a_j for all columns j, x the entries of column c below
+// the diagonal -- the norm (j = c), the reflector's application (j > c) and V's
+// Gram (j < c), since V = x / (alpha - beta) -- and the owner of row c that row.
+// Then T by workgroup 0, a thread per row of the recursion of
+// GenerateBlockTr("F","C") (Reflector.hpp:580-626).  False, with A untouched,
+// when a column's squared norm is outside [2^-600, 2^600] but not zero.
+// Bound by a grid-wide step per column, 6 us with three workgroups and 14 with
+// 160: 10000 x 100 takes 1.7 ms in all, 180 x 128 1.0, 779 x 55 0.46.  (One
+// workgroup alone, on the block in memory: 72, 2.0 and 1.2 ms; a column-wise
+// launch for 64 columns and less, without the attempt before it: 0.5 ms at
+// 90 x 90, where the attempt and this take 0.7.)
+// step: the first unused number of the grid-wide steps.  X, Y, M1, M2: scratch,
+// 64 x LDA_S each.
+__device__ __noinline__ bool blk_columnwise(CqrBlockArgs a, int step, LdsD* X, LdsD* Y, LdsD* M1, LdsD* M2) {
+  RNPX_CQR_GLOBAL(a);
+  const int tid = threadIdx.x, g = blockIdx.x, G = gridDim.x;
+  const int K = a.w, mp = a.mp;
+  const int j = tid & 127, half = tid >> 7, h0 = 32 * half, r0 = 64 * g + h0;  // this thread's column, its first row
+  double* Gm = a.scratch + kBG;
+  double y[32];
+#pragma unroll
+  for (int r = 0; r < 32; ++r)
+    y[r] = (r0 + r < mp && j < K) ? a.A[(size_t)(r0 + r) + (size_t)j * a.lda] : 0.0;
+  for (int c = -1; c < K; ++c) {  // c = -1: the columns' norms, which must be in range
+    double* slot = a.part + 256 * (c & 1);
+    double* rowc = a.scratch + kBRow + 128 * (c & 1);
+    LdsD* const xs = X + h0;
+    double d = 0.0, mx = 0.0;
+    if (c >= 0) {
+      double yc = 0.0;
+#pragma unroll
+      for (int r = 0; r < 32; ++r) {
+        if (j == c) xs[r] = r0 + r > c ? y[r] : 0.0;
+        if (r0 + r == c) yc = y[r];
+      }
+      if (c >= r0 && c < r0 + 32) store_through(rowc + j, yc);
+      __syncthreads();
+    }
+#pragma unroll
+    for (int r = 0; r < 32; ++r) {
+      const double x = c < 0 ? y[r] : xs[r];
+      d = fma(x, y[r], d);
+      mx = fmax(mx, fabs(x));
+    }
+    M1[tid] = d;
+    M1[256 + tid] = mx;
+    __syncthreads();
+    if (tid < 128) {
+      double* my = slot + (size_t)g * kBlkElems;
+      store_through(my + tid, M1[tid] + M1[128 + tid]);
+      if (c < 0 || tid == 0) store_through(my + 128 + tid, fmax(M1[256 + tid], M1[384 + tid]));
+    }
+    grid_step(a, step++, g, G, tid);
+    // the sum of a column's products (at c = -1 the largest entry beside it): two
+    // threads, every other workgroup's each, 16 loads in flight
+    d = mx = 0.0;
+    for (int q0 = half; q0 < G; q0 += 32) {
+      double v[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) v[u] = slot[(size_t)min(q0 + 2 * u, G - 1) * kBlkElems + j];
+#pragma unroll
+      for (int u = 0; u < 16; ++u)
+        if (q0 + 2 * u < G) d += v[u];
+    }
+    if (c < 0)
+      for (int q = half; q < G; q += 2) mx = fmax(mx, slot[(size_t)q * kBlkElems + 128 + j]);
+    else if (tid < G)
+      mx = slot[(size_t)tid * kBlkElems + 128];
+    const double rj = c >= 0 ? rowc[j] : 0.0;  // row c, column j
+    if (c >= 0) mx = wave_max(mx);
+    M1[tid] = d;
+    M1[256 + tid] = mx;
+    if (tid < 128) M1[512 + tid] = rj;
+    __syncthreads();
+    d = M1[j] + M1[128 + j];
+    if (c < 0) {
+      const double m = fmax(M1[256 + j], M1[384 + j]);
+      if (__syncthreads_or(!(d >= 0x1p-600 && d <= 0x1p600) && !(d == 0.0 && m == 0.0))) return false;
+      continue;
+    }
+    const double ss = M1[c] + M1[128 + c], alpha = M1[512 + c];
+    const double xmax = fmax(fmax(M1[256], M1[320]), fmax(M1[384], M1[448]));
+    double tau = 0.0, inv = 0.0;
+    if (ss >= 0x1p-600 && ss <= 0x1p600) {
+      double beta = hypot3(alpha, 0.0, sqrt(ss));
+      if (alpha > 0.0) beta = -beta;
+      tau = (beta - alpha) / beta;
+      inv = recip_t(alpha - beta);
+      const double cw = tau * fma(inv, d, rj);
+      const double diag = j == c ? beta : rj - cw;
+#pragma unroll
+      for (int r = 0; r < 32; ++r) {
+        const double v = xs[r] * inv;
+        if (j > c) y[r] -= v * cw;  // (xs is zero from row c up)
+        if (j == c && r0 + r > c) y[r] = v;
+        if (j >= c && r0 + r == c) y[r] = diag;
+      }
+    } else if (!(ss == 0.0 && xmax == 0.0)) {
+      return false;
+    }
+    if (g == 0) {
+      if (tid < c) Gm[tid * K + c] = fma(inv, d, rj);
+      if (tid == 0) a.tau[c] = tau;
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int r = 0; r < 32; ++r) {
+    const int gr = r0 + r;
+    if (gr < mp && j < K) {
+      a.A[(size_t)gr + (size_t)j * a.lda] = y[r];
+      a.V[(size_t)gr + (size_t)j * a.ldv] = (gr > j) ? y[r] : (gr == j ? 1.0 : 0.0);
+    }
+  }
+  if (g != 0) return true;
+  __syncthreads();
+  // T's row i by thread i: columns 0..63 in M1 (i < 64) or nowhere, 64..127 in M2 or X
+  LdsD* const lo = M1 + tid * LDA_S;
+  LdsD* const hi = (tid < NB ? M2 + tid * LDA_S : X + (tid & (NB - 1)) * LDA_S) - NB;
+  // (zeros left of the diagonal, so that every row's sum starts at column 0)
+  for (int e = tid; e < 64 * LDA_S; e += 256) M1[e] = M2[e] = X[e] = 0.0;
+  for (int c0 = 0; c0 < K; c0 += 32) {  // 32 columns of the Gram, then of T
+    __syncthreads();
+    for (int e = tid; e < 32 * 128; e += 256) {
+      const int c = c0 + e / 128, l = e % 128;
+      if (c < K) Y[e] = l < c ? Gm[l * K + c] : (l == c ? a.tau[c] : 0.0);
+    }
+    __syncthreads();
+    if (tid < 128)
+      for (int c = max(c0, tid); c < min(c0 + 32, K); ++c) {
+        LdsD* const gc = Y + (c - c0) * 128;
+        double s = 0.0, s2 = 0.0;
+        if (tid < NB)
+#pragma unroll 8
+          for (int l = 0; l < min(c, NB); ++l) s = fma(lo[l], gc[l], s);
+        if (c > NB)
+#pragma unroll 8
+          for (int l = NB; l < c; ++l) s2 = fma(hi[l], gc[l], s2);
+        (c < NB ? lo : hi)[c] = (tid == c) ? gc[c] : -gc[c] * (s + s2);
+      }
+  }
+  __syncthreads();
+  if (tid < K)
+    for (int c = 0; c < K; ++c)
+      a.T[(size_t)tid + (size_t)c * a.ldt] = (tid > c) ? 0.0 : (c < NB ? lo : hi)[c];
+  return true;
+}
+
+// What every workgroup does with a rejected block.
+__device__ __noinline__ void blk_rejected(CqrBlockArgs a, int step, LdsD* X, LdsD* Y, LdsD* M1, LdsD* M2, double* sh) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *a.fail = 1u;
+  if (!blk_columnwise(a, step, X, Y, M1, M2) && blockIdx.x == 0) blk_refactor(a, sh, threadIdx.x);
 }
 
 // T = -U D Z^T (upper) from U in M1 (on and above the diagonal), D in dcol and
@@ -885,6 +1045,11 @@ __global__ __launch_bounds__(256) void cqr_block_kernel(CqrBlockArgs a) {
   const bool two = w2 > 0;
   double* sc = a.scratch;
   double* part = a.part + (size_t)g * kBlkElems;
+  // step: the first grid-wide step not taken yet, the same in every workgroup
+  auto rejected = [&](int step) {
+    __syncthreads();
+    blk_rejected(a, step, (LdsD*)&Ab1[0][0], (LdsD*)&Ab2[0][0], (LdsD*)&M1[0][0], (LdsD*)&M2[0][0], rowbuf);
+  };
 
   // Both halves' rows of this workgroup, zero outside the block.
   {
@@ -920,6 +1085,12 @@ __global__ __launch_bounds__(256) void cqr_block_kernel(CqrBlockArgs a) {
     double* rp = sc + kBR + (size_t)3 * 4096 * pass;
     const bool is_first = pass > 0 && dev <= kFirstOrder;
     bool ok = pass == 0 || (dev <= kThirdPass && (is_first || pass < kBlkPasses));
+    // A zero tail in the first column (triangular, diagonal input) would reject
+    // the block in the reconstruction, some 170 us later.
+    if (pass == 0 && (a.zero_tails & 1)) {
+      const double d0 = gs[0], a0 = a.A[0];
+      ok = !(d0 - a0 * a0 <= 0x1p-42 * d0);
+    }
 #pragma unroll 1
     for (int half = 0; half < (two ? 2 : 1) && ok; ++half) {
       const bool first = one_copy(is_first), second_half = one_copy(half != 0), keep = one_copy(g == 2);
@@ -966,7 +1137,7 @@ __global__ __launch_bounds__(256) void cqr_block_kernel(CqrBlockArgs a) {
       if (ok) times_upper<64>(second_half ? Ab2 : Ab1, Xi, lane, wave);
     }
     if (!ok) {
-      if (g == 0) blk_refactor(a, rowbuf, tid);
+      rejected(2 * pass + 3);
       return;
     }
     np = pass + 1;
@@ -975,7 +1146,6 @@ __global__ __launch_bounds__(256) void cqr_block_kernel(CqrBlockArgs a) {
 
   // ---- 3: reconstruction ----
   const int last = (mp == w) ? w - 1 : -1;  // the column without a reflector
-  const double pmax = a.zero_tails ? 1.0 - 0x1p-40 : 2.0;
   f64x4 racc[3][4];
   if (g == 2) {
     // R's product of the passes' factors, in place of the first one's
@@ -1030,12 +1200,13 @@ __global__ __launch_bounds__(256) void cqr_block_kernel(CqrBlockArgs a) {
       for (int e = tid; e < NB * NB; e += 256) M1[e / NB][e % NB] = Ab[e / NB][e % NB];
       __syncthreads();
       // M1 = U and L, M2 = U^-1
-      const bool fits = small64::lu64<LDA_S>(&M1[0][0], rowbuf, &M2[0][0], tmpb, &okf, tid, lasth, pmax);
+      const bool fits = small64::lu64<LDA_S>(&M1[0][0], rowbuf, &M2[0][0], tmpb, &okf, tid, lasth,
+                                                  ((a.zero_tails >> half) & 1) ? 1.0 - 0x1p-40 : 2.0);
       save64(M2, ui, tid);
       if (tid < NB) dd[tid] = rowbuf[tid];
       publish(pub, fits ? 1u : kRejected);
       if (!fits) {
-        if (g == 0) blk_refactor(a, rowbuf, tid);
+        rejected(2 * np + 1);
         return;
       }
       for (int e = tid; e < NB * NB; e += 256) {
@@ -1066,7 +1237,7 @@ __global__ __launch_bounds__(256) void cqr_block_kernel(CqrBlockArgs a) {
         }
       // A only once the second half is accepted too
       if (fh && wait_verdict(&a.sync[kBlkPub2], a.abortf, &slot) == kRejected) {
-        blk_refactor(a, rowbuf, tid);
+        rejected(2 * np + 1);
         return;
       }
       for (int e = tid; e < NB * NB; e += 256) {
@@ -1111,7 +1282,10 @@ __global__ __launch_bounds__(256) void cqr_block_kernel(CqrBlockArgs a) {
       return;
     }
     if (g < half) return;  // (workgroup 0 left above)
-    if (wait_verdict(pub, a.abortf, &slot) == kRejected) return;
+    if (wait_verdict(pub, a.abortf, &slot) == kRejected) {
+      rejected(2 * np + 1);
+      return;
+    }
     load64(ui, M2, tid);
     __syncthreads();
     times_upper<64>(Ab, M2, lane, wave);  // V rows of this half

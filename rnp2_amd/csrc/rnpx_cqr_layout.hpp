@@ -16,9 +16,12 @@ constexpr int kU1i = kR + kRSize, kU12 = kU1i + kHalf, kT1 = kU12 + kHalf, kU2i 
 // their own, since nothing orders them after workgroup 2's stores into kR -- a
 // line of those that its cache writes back late would land on them.
 constexpr int kGram = kPublishedEnd, kTFactor = kGram + 128 * 128;
-constexpr int kScratch = kTFactor + 128 * 128;
+// a column's row of the block on its way to every workgroup, two parities
+constexpr int kRow = kTFactor + 128 * 128;
+constexpr int kScratch = kRow + 2 * 128;
 
-static_assert(kR + kRSize <= kU1i && kPublishedEnd <= kGram && kGram + 128 * 128 <= kTFactor,
+static_assert(kR + kRSize <= kU1i && kPublishedEnd <= kGram && kGram + 128 * 128 <= kTFactor &&
+                  kTFactor + 128 * 128 <= kRow,
               "block scratch regions overlap");
 
 }  // namespace blk

@@ -253,12 +253,12 @@ hipError_t launch_cqr_panel(const CqrArgs& a, int G, int rw, hipStream_t st);
 // CholeskyQR2 and Householder reconstruction.  Outputs: R and V packed in A,
 // tau (w), the block's clean V (ldv >= mp, zeros above the second 64 columns)
 // and T (w x w; 128 columns of ldt >= 128 are written).  If the block is
-// rejected, A is untouched until workgroup 0 refactors it column by column in
+// rejected, A is untouched until the workgroups refactor it column by column in
 // the same launch (*fail = 1).  G workgroups of 64 rows, at least three, all
 // resident at once (they meet at grid-wide reductions).
 struct CqrBlockArgs {
   int mp, w;            // block rows and columns (w <= 128, w <= mp)
-  bool zero_tails;      // columns with exact zeros below the diagonal get tau = 0 (column by column)
+  int zero_tails;       // halves (bits 0, 1) whose columns with exact zeros below the diagonal get tau = 0 (column by column)
   double* A; long lda;  // block top-left
   double* tau;          // out: w scalars
   double* V; long ldv;  // out: clean V, mp x w

@@ -761,7 +761,7 @@ int geqrf_dev(Handle* h, int m, int n, T* A, long lda, T* tau, T* B, int nrhs, l
         ba.w = w;
         // Short and ragged blocks (small matrices, factorizations' ends) keep
         // the reference's tau = 0 for zero tails; full ones, as ever, tau = 2.
-        ba.zero_tails = w < 2 * nb || m - i < 3 * nb;
+        ba.zero_tails = w < 2 * nb || m - i < 3 * nb ? 3 : 0;
         ba.A = A + (size_t)i + (size_t)i * lda;
         ba.lda = lda;
         ba.tau = tau + i;

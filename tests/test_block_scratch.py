@@ -20,6 +20,7 @@ int main() {
   std::printf("published %d %d\\n", kU1i, kPublishedEnd - kU1i);
   std::printf("gram %d %d\\n", kGram, 128 * 128);
   std::printf("tfactor %d %d\\n", kTFactor, 128 * 128);
+  std::printf("row %d %d\\n", kRow, 2 * 128);
   std::printf("all 0 %d\\n", kScratch);
 }
 """
@@ -40,5 +41,5 @@ def test_regions_are_disjoint(tmp_path):
 
 def test_kernel_takes_its_offsets_from_the_layout():
     s = open(os.path.join(CSRC, "rnpx_cqr.hip")).read()
-    for name, field in (("kBR", "kR"), ("kBU1i", "kU1i"), ("kBD2", "kD2"), ("kBG", "kGram"), ("kBTF", "kTFactor")):
+    for name, field in (("kBR", "kR"), ("kBU1i", "kU1i"), ("kBD2", "kD2"), ("kBG", "kGram"), ("kBTF", "kTFactor"), ("kBRow", "kRow")):
         assert f"{name} = blk::{field}" in s

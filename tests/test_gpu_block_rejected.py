@@ -1,0 +1,89 @@
+"""Blocks that the outer-block kernel rejects and refactors column by column
+(every workgroup its 64 rows, a grid-wide step per column), against the oracle:
+exact zeros below the diagonal in short blocks and ragged halves (tau = 0,
+Reflector.hpp:122-125), blocks too ill conditioned for CholeskyQR, zero columns,
+and norms that need Generate's scaling.  Bar: the factorization tests' (R, tau, V
+to 1e-11 of the column scale); for ill-conditioned blocks, whose R is only
+determined to eps * condition, residual and orthogonality <= 10 n eps."""
+import time
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+import rnp2_amd as R
+from metrics import orth_error, qr_residual, rel_err_colscaled
+
+pytestmark = pytest.mark.gpu
+
+
+def check(a, elementwise=True):
+    m, n = a.shape
+    k = min(m, n)
+    af, tau = R.factor(a)
+    r = np.triu(af[:k])
+    q = R.generateq(af[:, :k], tau, n=k)
+    assert qr_residual(a, q, r) <= 10 and orth_error(q) <= 10
+    if elementwise:
+        af_o, tau_o = O.factor(a)
+        assert np.array_equal(tau == 0, tau_o == 0)
+        assert rel_err_colscaled(r, np.triu(af_o[:k])) <= 1e-11
+        assert np.max(np.abs(tau - tau_o)) <= 1e-11
+        assert np.max(np.abs(np.tril(af, -1) - np.tril(af_o, -1))) <= 1e-9
+
+
+def zero_tails_from(m, n, j):
+    """Columns from j on have exact zeros below the diagonal, and still do when
+    the reflectors of the columns before, dense in the first j rows, are through."""
+    rng = np.random.default_rng(m + n + j)
+    a = np.triu(rng.standard_normal((m, n))) / n + 2.0 * np.eye(m, n)
+    a[:j, :j] = rng.standard_normal((j, j)) / n + np.eye(j)
+    return a
+
+
+# three workgroups and many; one half and two, short blocks and tall ones
+@pytest.mark.parametrize("m,n,j", [(16, 16, 0), (20, 17, 3), (64, 64, 10), (65, 64, 63), (90, 90, 0), (100, 81, 70),
+                                   (130, 128, 64), (191, 128, 1), (192, 55, 0), (700, 55, 20), (4000, 33, 32),
+                                   (192, 100, 66), (3000, 127, 90), (9001, 100, 70), (16384, 90, 80)])
+def test_zero_tails(m, n, j):
+    check(zero_tails_from(m, n, j))
+
+
+@pytest.mark.parametrize("m,n", [(70, 64), (150, 128), (800, 40), (5000, 128), (16384, 128)])
+@pytest.mark.parametrize("kind", ["ill", "zero columns", "small", "large"])
+def test_other_rejected_blocks(m, n, kind):
+    rng = np.random.default_rng(m + n)
+    a = rng.standard_normal((m, n))
+    if kind == "ill":
+        u = np.linalg.qr(a)[0]
+        v = np.linalg.qr(rng.standard_normal((n, n)))[0]
+        a = u * np.logspace(0, -13, n) @ v
+    elif kind == "zero columns":
+        a[:, [0, n // 2, n - 1]] = 0.0
+    else:  # one column's squared norm leaves [2^-600, 2^600]
+        a[:, n // 3] *= 2.0 ** (-330 if kind == "small" else 330)
+    check(a, elementwise=kind in ("small", "large"))
+
+
+@pytest.mark.parametrize("m,n,j", [(10000, 32, 5), (10000, 100, 70), (16384, 127, 64)])
+def test_cost_of_a_rejection(m, n, j):
+    """A rejected block costs a grid-wide step per column: 30 us each at most (10
+    to 15 measured; one workgroup alone took 200 to 1000)."""
+    h = R.Handle()
+    tau = torch.empty(n, dtype=torch.float64, device="cuda")
+    best = []
+    for a in (np.random.default_rng(0).standard_normal((m, n)), zero_tails_from(m, n, j)):
+        A0, A = (R.colmajor_empty(m, n, torch.float64) for _ in range(2))
+        A0.copy_(torch.from_numpy(a).cuda())
+        ts = []
+        for _ in range(6):
+            A.copy_(A0)
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            h.geqrf(A, tau)
+            h.synchronize()
+            ts.append(time.perf_counter() - t)
+        best.append(min(ts))
+    h.close()
+    assert best[1] - best[0] <= 30e-6 * n, best
