@@ -759,9 +759,10 @@ int geqrf_dev(Handle* h, int m, int n, T* A, long lda, T* tau, T* B, int nrhs, l
         CqrBlockArgs ba;
         ba.mp = m - i;
         ba.w = w;
-        // Short and ragged blocks (small matrices, factorizations' ends) keep
-        // the reference's tau = 0 for zero tails; full ones, as ever, tau = 2.
-        ba.zero_tails = w < 2 * nb || m - i < 3 * nb ? 3 : 0;
+        // Short blocks and ragged halves (small matrices, factorizations' ends)
+        // keep the reference's tau = 0 for zero tails; full halves of 64 columns
+        // take tau = 2 there, which the reconstruction gives them.
+        ba.zero_tails = m - i < 3 * nb ? 3 : w < nb ? 1 : w > nb && w < 2 * nb ? 2 : 0;
         ba.A = A + (size_t)i + (size_t)i * lda;
         ba.lda = lda;
         ba.tau = tau + i;

@@ -66,24 +66,47 @@ def test_other_rejected_blocks(m, n, kind):
     check(a, elementwise=kind in ("small", "large"))
 
 
+def seconds(a):
+    m, n = a.shape
+    h = R.Handle()
+    A0, A = (R.colmajor_empty(m, n, torch.float64) for _ in range(2))
+    A0.copy_(torch.from_numpy(a).cuda())
+    tau = torch.empty(n, dtype=torch.float64, device="cuda")
+    ts = []
+    for _ in range(6):
+        A.copy_(A0)
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        h.geqrf(A, tau)
+        h.synchronize()
+        ts.append(time.perf_counter() - t)
+    h.close()
+    return min(ts)
+
+
 @pytest.mark.parametrize("m,n,j", [(10000, 32, 5), (10000, 100, 70), (16384, 127, 64)])
 def test_cost_of_a_rejection(m, n, j):
     """A rejected block costs a grid-wide step per column: 30 us each at most (10
     to 15 measured; one workgroup alone took 200 to 1000)."""
-    h = R.Handle()
-    tau = torch.empty(n, dtype=torch.float64, device="cuda")
-    best = []
-    for a in (np.random.default_rng(0).standard_normal((m, n)), zero_tails_from(m, n, j)):
-        A0, A = (R.colmajor_empty(m, n, torch.float64) for _ in range(2))
-        A0.copy_(torch.from_numpy(a).cuda())
-        ts = []
-        for _ in range(6):
-            A.copy_(A0)
-            torch.cuda.synchronize()
-            t = time.perf_counter()
-            h.geqrf(A, tau)
-            h.synchronize()
-            ts.append(time.perf_counter() - t)
-        best.append(min(ts))
-    h.close()
+    best = [seconds(a) for a in (np.random.default_rng(0).standard_normal((m, n)), zero_tails_from(m, n, j))]
     assert best[1] - best[0] <= 30e-6 * n, best
+
+
+@pytest.mark.parametrize("m,n,j", [(10000, 100, 20), (3000, 64, 63), (3000, 80, 0)])
+def test_short_tail_in_a_full_half_is_no_rejection(m, n, j):
+    """One column of the first 64 whose entries below the diagonal are 1e-9 of its
+    norm once the columns before are through: a tall matrix keeps the fast path
+    (its reflector, tau = 2 to rounding, is what the reference has there)."""
+    rng = np.random.default_rng(n)
+    a = rng.standard_normal((m, n))
+    base = seconds(a)
+    af, tau = O.factor(a[:, :j]) if j else (a[:, :0], [])
+    x = np.zeros(m)
+    x[j] = 1.0
+    x[j + 1:] = 1e-9 * rng.standard_normal(m - j - 1) / np.sqrt(m)
+    for i in reversed(range(j)):  # column j as the reflectors before it turn into x
+        v = np.concatenate([np.zeros(i), [1.0], af[i + 1:, i]])
+        x -= tau[i] * v * (v @ x)
+    a[:, j] = x
+    check(a)
+    assert seconds(a) <= 1.5 * base
