@@ -497,7 +497,12 @@ __global__ __launch_bounds__(256) void cqr_panel_kernel(CqrArgs a) {
 //      up to about 1e7; CholeskyQR iterated).  Otherwise the block is
 //      rejected, as it is when a pivot falls below 2^-40 of its column's
 //      squared norm, a squared norm is outside [2^-600, 2^600] or a value is
-//      not finite.  Every workgroup takes the same decision from the same
+//      not finite.  A pivot of the second half may fall that low because its
+//      columns lie near the first half's span (collinear regressors), which
+//      says nothing about their part outside it: A2 - Q1 R12 then goes into the
+//      next pass as it is (R22 = I), up to twice (what is left along Q1 after one
+//      projection, the first half's loss of orthogonality, can still be the
+//      larger part), and is held against its own norms there.  Every workgroup takes the same decision from the same
 //      reduced Gram, and A is untouched until the block is accepted; a rejected
 //      block is refactored column by column (blk_columnwise).
 //   3. Reconstruction [Q1 Q2] - [D; 0] = L U without another reduction:
@@ -539,6 +544,9 @@ constexpr int kCross = 16 * 256;                   // a 64x64 product in 16 tile
 constexpr int kBlkElems = kCqrBlockPart;           // upper tiles of a 128x128 Gram: G11, G12, G22
 static_assert(2 * kGramElems + kCross == kBlkElems, "Gram layout: tiles 0..9, 10..25, 26..35");
 constexpr int kBlkPasses = blk::kPasses;
+// a second half may be projected without being normalized in the passes before
+// this one (two passes are left to normalize it and to see that it is)
+constexpr int kBlkProject = kBlkPasses - 2;
 constexpr double kThirdPass = 0x1p-3;
 constexpr unsigned kRejected = 2u;                 // flag value: the block goes column by column
 constexpr int kBR = blk::kR, kBU1i = blk::kU1i, kBU12 = blk::kU12, kBT1 = blk::kT1, kBU2i = blk::kU2i,
@@ -1073,6 +1081,7 @@ __global__ __launch_bounds__(256) void cqr_block_kernel(CqrBlockArgs a) {
 
   // ---- 1 and 2: passes; workgroup 2 keeps their factors for R ----
   int np = 0;  // passes done (factors at sc + kBR + 3 * 4096 * pass)
+  bool later = false;  // the second half is projected only so far (R22 = I)
 #pragma unroll 1
   for (int pass = 0;; ++pass) {
     blk_gram(Ab1, Ab2, two, part, lane, wave);
@@ -1081,10 +1090,11 @@ __global__ __launch_bounds__(256) void cqr_block_kernel(CqrBlockArgs a) {
     BlkGram gm;
     read_gram(gs, two, gm, tid);
     double dev = 1.0;
-    if (pass > 0) dev = blk_dev(gm, w, red4, tid);
+    if (pass > 0) dev = blk_dev(gm, later ? NB : w, red4, tid);
     double* rp = sc + kBR + (size_t)3 * 4096 * pass;
     const bool is_first = pass > 0 && dev <= kFirstOrder;
-    bool ok = pass == 0 || (dev <= kThirdPass && (is_first || pass < kBlkPasses));
+    const bool was_later = later;
+    bool ok = pass == 0 || (dev <= kThirdPass && ((is_first && !later) || pass < kBlkPasses));
     // A zero tail in the first column (triangular, diagonal input) would reject
     // the block in the reconstruction, some 170 us later.
     if (pass == 0 && (a.zero_tails & 1)) {
@@ -1093,7 +1103,7 @@ __global__ __launch_bounds__(256) void cqr_block_kernel(CqrBlockArgs a) {
     }
 #pragma unroll 1
     for (int half = 0; half < (two ? 2 : 1) && ok; ++half) {
-      const bool first = one_copy(is_first), second_half = one_copy(half != 0), keep = one_copy(g == 2);
+      const bool first = one_copy(is_first && !(half != 0 && was_later)), second_half = one_copy(half != 0), keep = one_copy(g == 2);
       double(*X)[LDA_S] = second_half ? M2 : M1;   // the Gram, then R
       double(*Xi)[LDA_S] = second_half ? M1 : M2;  // R^-1
       f64x4 acc[4];
@@ -1131,6 +1141,15 @@ __global__ __launch_bounds__(256) void cqr_block_kernel(CqrBlockArgs a) {
         __syncthreads();
       } else {
         ok = small64::chol64<LDA_S>(&X[0][0], &Xi[0][0], tmpb, gdiag, &okf, tid);
+        if (second_half) {
+          later = !ok && pass < kBlkProject;
+          if (later) {
+            ok = true;
+            if (keep)
+              for (int e = tid; e < NB * NB; e += 256) rs[e] = (e / NB == e % NB) ? 1.0 : 0.0;
+            continue;
+          }
+        }
         if (ok && keep)
           for (int e = tid; e < NB * NB; e += 256) rs[e] = (e / NB <= e % NB) ? X[e / NB][e % NB] : 0.0;
       }
@@ -1141,7 +1160,7 @@ __global__ __launch_bounds__(256) void cqr_block_kernel(CqrBlockArgs a) {
       return;
     }
     np = pass + 1;
-    if (pass > 0 && dev <= kSecondPass) break;  // orthonormal to working precision now
+    if (pass > 0 && dev <= kSecondPass && !was_later && !later) break;  // orthonormal to working precision now
   }
 
   // ---- 3: reconstruction ----

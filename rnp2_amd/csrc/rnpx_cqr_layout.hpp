@@ -6,7 +6,7 @@ namespace rnpx {
 namespace blk {
 
 constexpr int kHalf = 64 * 64;                     // a 64 x 64 block
-constexpr int kPasses = 3;                         // Cholesky passes at most (and one first-order pass)
+constexpr int kPasses = 4;                         // Cholesky passes at most (and one first-order pass)
 // R11, R12, R22 of each pass (workgroup 2)
 constexpr int kR = 0, kRSize = 3 * kHalf * (kPasses + 1);
 // the blocks that one workgroup publishes to the others

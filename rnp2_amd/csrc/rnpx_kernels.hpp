@@ -264,7 +264,7 @@ struct CqrBlockArgs {
   double* V; long ldv;  // out: clean V, mp x w
   double* T; long ldt;  // out: T
   double* part;         // scratch: G * kCqrBlockPart (each workgroup's partial Gram)
-  double* gsum;         // scratch: 4 * kCqrBlockPart (the reduced Gram of each pass)
+  double* gsum;         // scratch: kCqrBlockGrams * kCqrBlockPart (the reduced Gram of each pass)
   double* scratch;      // scratch: kCqrBlockScratch doubles
   unsigned* sync;       // kCqrBlockSyncWords words, zero at launch
   unsigned* abortf;     // sticky error flag
@@ -272,6 +272,7 @@ struct CqrBlockArgs {
 };
 constexpr int kCqrBlockSyncWords = 256;
 constexpr int kCqrBlockScratch = blk::kScratch;
+constexpr int kCqrBlockGrams = blk::kPasses + 1;
 constexpr int kCqrBlockPart = 36 * 256;  // the upper 16 x 16 tiles of a 128 x 128 Gram
 // Workgroups for an mp-row, w-column block, 0 when the block kernel does not apply.
 int cqr_block_groups(int mp, int w, int max_groups);

@@ -703,7 +703,7 @@ int geqrf_dev(Handle* h, int m, int n, T* A, long lda, T* tau, T* B, int nrhs, l
   if (use_block) {
     const std::pair<Buffer*, size_t> need[] = {
         {&h->cqr_part, sizeof(double) * (size_t)std::max(3, (m + 63) / 64) * kCqrBlockPart},
-        {&h->cqr_gsum, sizeof(double) * 4 * kCqrBlockPart},
+        {&h->cqr_gsum, sizeof(double) * kCqrBlockGrams * kCqrBlockPart},
         {&h->cqr_scratch, sizeof(double) * kCqrBlockScratch}};
     const int s = reserve(h, need, 3);
     if (s == RNPX_ERR_NOMEM) use_block = false;

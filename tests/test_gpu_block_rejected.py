@@ -110,3 +110,31 @@ def test_short_tail_in_a_full_half_is_no_rejection(m, n, j):
     a[:, j] = x
     check(a)
     assert seconds(a) <= 1.5 * base
+
+
+@pytest.mark.parametrize("m,n", [(130, 128), (200, 100), (3000, 128), (2000, 256), (16384, 128)])
+@pytest.mark.parametrize("eps", [1e-5, 1e-7, 1e-9, 1e-12, 1e-15, 0.0])
+def test_second_half_near_the_first_halfs_span(m, n, eps):
+    """Collinear regressors: the second 64 columns of a block are combinations of
+    the first 64 plus eps noise.  Residual and orthogonality at the bar; the block
+    takes one or two passes more (50 us each) instead of a column-wise
+    refactorization (1 ms and more)."""
+    rng = np.random.default_rng(m)
+    a = rng.standard_normal((m, n))
+    base = seconds(a)
+    for i in range(0, n, 128):
+        e = min(i + 128, n)
+        a[:, i + 64:e] = a[:, i:i + 64] @ rng.standard_normal((64, e - i - 64)) / 8 + eps * a[:, i + 64:e]
+    check(a, elementwise=False)
+    assert seconds(a) <= 1.7 * base + 100e-6 * (n // 128)
+
+
+def test_second_half_near_a_badly_conditioned_first_half():
+    """The first half at condition 1e4: one projection leaves 1e-8 of the second
+    half along it, more than the 1e-11 that is to be found outside."""
+    rng = np.random.default_rng(5)
+    u = np.linalg.qr(rng.standard_normal((3000, 64)))[0]
+    v = np.linalg.qr(rng.standard_normal((64, 64)))[0]
+    a1 = u * np.logspace(0, -4, 64) @ v
+    check(np.hstack([a1, a1 @ rng.standard_normal((64, 64)) + 1e-11 * rng.standard_normal((3000, 64))]),
+          elementwise=False)
