@@ -16,7 +16,7 @@ struct Handle;
 struct Buffer {
   void* p = nullptr;
   size_t bytes = 0;
-  hipError_t ensure(size_t b, Handle* h);
+  hipError_t ensure(size_t b, Handle* h, bool exact = false);
   void release();
 };
 
@@ -89,6 +89,11 @@ struct Handle {
             &cqr_scratch, &wbuf2, &zbuf2, &part2, &misc2, &trsm_flags, &lqbuf, &qlbuf, &lubuf, &lull, &rfbuf, &invbuf, &exbuf, &exsave, &rinv, &zcqr, &gemvbuf};
   }
   hipError_t sync_all_streams();       // the handle's stream, panel stream and partition streams
+  // The outer-block kernel's buffers, which a call can do without (panel by
+  // panel): given back where a handle's budget has no room for something else,
+  // unless a factorization is using them.
+  bool block_busy = false;
+  bool give_back_block();
   void* batch = nullptr;               // batched-call descriptor buffers
   void (*batch_free)(void*) = nullptr;
   int update_prec = 0;                 // 1: trailing-update products on FP32 MFMA

@@ -293,13 +293,13 @@ hipError_t launch_tfactor(const T* gram, int ldg, int k, int nb, T* Tout, int ld
 // The T factors of a stored factorization, all w-column blocks (w 32, 64 or
 // 128) of k reflectors at once.  launch_gram_blocks: gram[b] (w x w, blocks w*w
 // apart) in the layout launch_tfactor reads, from the clean V (n x k, zeros
-// above the unit diagonal) and tau; part holds gram_blocks_slices(n, k, w) *
+// above the unit diagonal) and tau; part holds gram_blocks_slices(n, k, w, most) *
 // ceil(k / w) * w * w elements, the slices added in order.  launch_tfactor_blocks:
 // T[b] (w x w) from gram[b]; at w = 128 its two 64-column diagonal parts (zero
 // elsewhere), to be joined by T12 = -T11 gram12 T22.
-int gram_blocks_slices(int n, int k, int w, int* kslice);
+int gram_blocks_slices(int n, int k, int w, int most, int* kslice);
 template <typename T>
-hipError_t launch_gram_blocks(int n, int k, int w, const T* V, long ldv, const T* tau, T* gram, T* part,
+hipError_t launch_gram_blocks(int n, int k, int w, int most, const T* V, long ldv, const T* tau, T* gram, T* part,
                               hipStream_t st);
 template <typename T>
 hipError_t launch_tfactor_blocks(const T* gram, int w, int k, T* Tout, hipStream_t st);

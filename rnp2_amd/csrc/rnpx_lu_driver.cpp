@@ -33,11 +33,12 @@ int getrf_dev(Handle* h, int m, int n, T* A, long lda, int* piv_host, int* info)
   if (rw == 0) return RNPX_ERR_UNSUPPORTED;
   // scratch: per panel the zero-pivot column, the relative pivots and the
   // moved rows (ints); complex panels' candidates, row c and sync words
-  const size_t nd = S<T>::cplx ? (size_t)2 * 256 * kLuPartPerGroup + 4 * nb + 2 * nb : 0;
+  const size_t groups = (size_t)(m + rw - 1) / rw;
+  const size_t nd = S<T>::cplx ? 2 * groups * kLuPartPerGroup + 4 * nb + 2 * nb : 0;
   const size_t nints = (size_t)npan + k + (size_t)npan * kLuMoveWords;
   RNPX_TRY(h->lubuf.ensure(sizeof(double) * nd + sizeof(unsigned) * 2 * nb + sizeof(int) * nints, h));
   double* part = (double*)h->lubuf.p;
-  double* rowc = part + (size_t)2 * 256 * kLuPartPerGroup;
+  double* rowc = part + 2 * groups * kLuPartPerGroup;
   unsigned* sync = (unsigned*)(part + nd);
   int* zl = (int*)(sync + 2 * nb);
   int* prel = zl + npan;

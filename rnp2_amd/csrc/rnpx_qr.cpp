@@ -16,9 +16,15 @@ namespace rnpx {
 // ---------------------------------------------------------------------------
 // Workspace
 // ---------------------------------------------------------------------------
-hipError_t Buffer::ensure(size_t b, Handle* h) {
+hipError_t Buffer::ensure(size_t b, Handle* h, bool exact) {
   if (b <= bytes) return hipSuccess;
-  if (h && h->budget && h->held_bytes() - bytes + b > h->budget) return hipErrorOutOfMemory;
+  size_t most = (size_t)-1;
+  if (h && h->budget) {
+    if (h->held_bytes() - bytes + b > h->budget) (void)h->give_back_block();
+    const size_t others = h->held_bytes() - bytes;
+    if (others + b > h->budget) return hipErrorOutOfMemory;
+    most = h->budget - others;
+  }
   if (p) {
     // The buffer may be in use on any stream of the handle (the look-ahead's
     // panel stream grows its GEMM scratch while earlier panel work is queued):
@@ -29,7 +35,7 @@ hipError_t Buffer::ensure(size_t b, Handle* h) {
     p = nullptr;
     bytes = 0;
   }
-  size_t want = b + (b >> 3);  // grow with some headroom
+  const size_t want = exact ? b : std::min(b + (b >> 3), most);  // grow with some headroom
   hipError_t e = hipMalloc(&p, want);
   if (e != hipSuccess) {
     p = nullptr;
@@ -38,15 +44,32 @@ hipError_t Buffer::ensure(size_t b, Handle* h) {
   bytes = want;
   return hipSuccess;
 }
+bool Handle::give_back_block() {
+  Buffer* const bufs[] = {&cqr_part, &cqr_gsum, &cqr_scratch};
+  size_t had = 0;
+  for (Buffer* b : bufs) had += b->bytes;
+  if (block_busy || had == 0 || sync_all_streams() != hipSuccess) return false;
+  for (Buffer* b : bufs) b->release();
+  return true;
+}
+
 // Grow every buffer to what is needed, or none: RNPX_ERR_NOMEM, the buffers
 // that did grow given back, when the budget or the device does not hold all.
+// (The headroom of the larger ones must not take a smaller one's room: where
+// the budget holds no headroom at all, they grow to what is needed.)
 static int reserve(Handle* h, const std::pair<Buffer*, size_t>* need, int count) {
-  size_t total = h->held_bytes();
-  for (int i = 0; i < count; ++i)
-    if (need[i].second > need[i].first->bytes) total += need[i].second - need[i].first->bytes;
-  if (h->budget && total > h->budget) return RNPX_ERR_NOMEM;
+  auto total = [&](int headroom) {
+    size_t t = h->held_bytes();
+    for (int i = 0; i < count; ++i) {
+      const size_t b = need[i].second, has = need[i].first->bytes;
+      if (b > has) t += b + (headroom ? b >> 3 : 0) - has;
+    }
+    return t;
+  };
+  if (h->budget && total(0) > h->budget && !(h->give_back_block() && total(0) <= h->budget)) return RNPX_ERR_NOMEM;
+  const bool exact = h->budget && total(1) > h->budget;
   for (int i = 0; i < count; ++i) {
-    const hipError_t e = need[i].first->ensure(need[i].second, h);
+    const hipError_t e = need[i].first->ensure(need[i].second, h, exact);
     if (e == hipSuccess) continue;
     (void)hipGetLastError();
     RNPX_TRY(h->sync_all_streams());
@@ -336,7 +359,8 @@ static int pick_ksplit(const Handle* h, int rows, int cols_tiles) {
   // the narrow products (one or two column tiles) that sit on the chain of
   // panels, where latency matters more than the partial sums' traffic.
   int want = (cols_tiles <= 2 ? 1024 : 512) / std::max(1, cols_tiles);
-  int maxs = std::max(1, rows / (cols_tiles <= 2 ? 64 : 512));
+  // (128 rows a slice under a memory budget: the slices' sums are the scratch)
+  int maxs = std::max(1, rows / (cols_tiles <= 2 ? (h->budget ? 128 : 64) : 512));
   // narrow products: up to 64 slices (a tall panel's W is otherwise a long
   // chain of K slices on few workgroups)
   return std::max(1, std::min(want, std::min(maxs, cols_tiles <= 2 ? 64 : 32)));
@@ -424,15 +448,19 @@ static int apply_block_dev(Handle* h, char side, char trans, int mc, int nc, int
 // T block b at Tm + b w w: the Grams, the leaves' recurrence, and at w = 128
 // (real) the two leaves joined, T12 = -T11 (V1^T V2) T22; one launch each for
 // all blocks.  Scratch: gram (k/w blocks), misc (the Grams' slices), misc2.
+static int gram_most(const Handle* h, int n) {
+  // slices of a Gram: under a memory budget few and long ones
+  return h->budget ? std::max(1, std::min(64, n / 256)) : 96;
+}
 template <typename T>
 static int tfactor_blocks(Handle* h, int n, int k, int w, const T* V, long ldv, const T* tau, T* Tm) {
   int kslice = 0;
-  const int nblk = (k + w - 1) / w, ns = gram_blocks_slices(n, k, w, &kslice);
+  const int nblk = (k + w - 1) / w, most = gram_most(h, n), ns = gram_blocks_slices(n, k, w, most, &kslice);
   const size_t ws = (size_t)w * w;
   RNPX_TRY(h->gram.ensure(sizeof(T) * ws * nblk, h));
   RNPX_TRY(h->misc.ensure(sizeof(T) * ws * nblk * ns, h));
   T* G = (T*)h->gram.p;
-  RNPX_TRY(launch_gram_blocks<T>(n, k, w, V, ldv, tau, G, (T*)h->misc.p, h->stream));
+  RNPX_TRY(launch_gram_blocks<T>(n, k, w, most, V, ldv, tau, G, (T*)h->misc.p, h->stream));
   RNPX_TRY(launch_tfactor_blocks<T>(G, w, k, Tm, h->stream));
   if constexpr (!S<T>::cplx) {
     if (w == 128) {
@@ -467,7 +495,7 @@ template <typename T>
 static int wy_plan(Handle* h, bool own_v, bool left, int nq, int k, int rows, int cols, bool shrink, WyPlan* out) {
   // no wider than the reflectors: a T leaf of 64 complex columns takes 30 us where
   // one of 32 takes 15
-  const int wide = S<T>::cplx ? (k > 32 ? 64 : 32) : (k > 64 ? 128 : 64), narrow = S<T>::cplx ? 32 : 64;
+  const int wide = S<T>::cplx ? (k > 32 ? 64 : 32) : (k > 64 ? 128 : 64), narrow = pick_nb<T>(h, rows, cols);
   const int most = own_v ? std::min(k, 2048) : k;
   const WyPlan tries[3] = {{wide, (most + wide - 1) / wide * wide}, {wide, wide}, {narrow, narrow}};
   for (int t = h->budget ? 2 : 0; t < 3; ++t) {
@@ -475,14 +503,15 @@ static int wy_plan(Handle* h, bool own_v, bool left, int nq, int k, int rows, in
     const int cw = std::min(p.chunk, k), nblk = (cw + p.w - 1) / p.w;
     const size_t ws = sizeof(T) * (size_t)p.w * p.w;
     // slices of the Grams, of this chunk or a shorter last one
-    const int per = std::min(96, std::max(1, nq / 32));
+    const int per = std::min(gram_most(h, nq), std::max(1, nq / 32));
     const size_t nsl = std::min(per * nblk, std::max(nblk, 768 / (p.w <= 64 ? 1 : 4)));
     size_t wz = 0, part = 0;
     for (int i = 0; i < k; i += p.w) {
       const int mc = left ? rows - i : rows, nc = (left && !shrink) ? cols : cols - i;
       const int other = left ? nc : mc, ks = pick_ksplit(h, left ? mc : nc, (other + 127) / 128);
-      wz = std::max(wz, sizeof(T) * (size_t)p.w * other);
-      if (ks > 1) part = std::max(part, sizeof(T) * (size_t)ks * p.w * other);
+      const size_t ib = std::min(p.w, k - i);
+      wz = std::max(wz, sizeof(T) * ib * other);
+      if (ks > 1) part = std::max(part, sizeof(T) * (size_t)ks * ib * other);
     }
     const std::pair<Buffer*, size_t> need[] = {{&h->vbuf, own_v ? sizeof(T) * (size_t)nq * cw : 0},
                                                {&h->tbuf, ws * nblk},
@@ -671,6 +700,7 @@ int geqrf_dev(Handle* h, int m, int n, T* A, long lda, T* tau, T* B, int nrhs, l
   // rest is checked while the first panel runs, from a copy of those
   // columns that is put back if the factorization has to start over.
   auto factor_nonfinite = [&]() -> int {
+    h->block_busy = false;
     RNPX_CHECK(geqrf_exact<T>(h, m, n, A, lda, tau, h->exact_lwork));
     if (nrhs > 0) RNPX_CHECK(ormqr_dev<T>(h, 'L', 'C', m, nrhs, k, A, lda, tau, B, ldb));
     return RNPX_OK;
@@ -682,6 +712,99 @@ int geqrf_dev(Handle* h, int m, int n, T* A, long lda, T* tau, T* B, int nrhs, l
     RNPX_CHECK(any_nonfinite<T>(h, m, split_scan ? w0 : n, A, lda, &bad, st));
     if (bad) return factor_nonfinite();
   }
+  // Outer blocks in one launch (real, 64-column panels, 128-column blocks,
+  // tuning panel 0).
+  bool use_block = !S<T>::cplx && h->tune.panel == 0 && nb == 64 && nbo % (2 * nb) == 0 &&
+                   cqr_block_groups(m, std::min(nb, k), std::min(256, h->num_cus)) > 0;
+  static_assert(2 * kCqrSyncWords >= kCqrBlockSyncWords, "a block uses its two panels' sync words");
+  // (one panel's words more: a last block of one panel still uses two)
+  const int sync_words = 1 + 2 * npan + kCqrSyncWords * (npan + 1);
+  const size_t misc2_bytes = sizeof(T) * (size_t)std::max(3 * nb * nb, 2 * (nbo / 2) * (nbo / 2));
+  // An outer block of w columns is split into w1 = 2 nb (a block-kernel
+  // unit) or nb columns and the rest.
+  auto split_of = [&](int w) { return w > 2 * nb ? 2 * nb : nb; };
+  int pcus = h->tune.panel_cus;
+  if (pcus == 0) {
+    static const int env_cus = [] {
+      const char* e = getenv("RNPX_PANEL_CUS");
+      return e ? atoi(e) : 0;
+    }();
+    pcus = env_cus;
+  }
+  const bool partition = look && pcus > 0 && G0 <= pcus && !h->ext_pstream;
+  int cg = 0, crw = 0;
+  // the 64-column CholeskyQR2 panels' buffers (later panels may use more, smaller
+  // workgroups than the first)
+  const bool cqr = use_cqr<T>(h, m, std::min(nb, k), nb, &cg, &crw);
+  const size_t cqr_groups = std::min(std::min(kCqrMaxGroups, h->num_cus), (m + 63) / 64);
+  size_t part_b = cqr ? sizeof(double) * cqr_groups * 2560 : 0;
+  size_t gsum_b = cqr ? sizeof(double) * (2 + 16) * 2560 : 0;  // gsum, then group sums
+  size_t scratch_b = cqr ? sizeof(double) * kCqrScratch : 0;
+  // Everything the call needs, block by block or panel by panel: in a handle's
+  // budget the block kernel's buffers, 72 KB per 64 rows, must not take the
+  // products' room.
+  auto reserve_all = [&](bool block) -> int {
+    size_t wz[2] = {0, 0}, part[2] = {0, 0};  // the products' scratch: main stream, panel stream
+    auto product = [&](int q, int rows, int nc, int kk) {
+      if (rows <= 0 || nc <= 0 || kk <= 0) return;
+      const int ks = pick_ksplit(h, rows, (nc + 127) / 128);
+      wz[q] = std::max(wz[q], sizeof(T) * (size_t)kk * nc);
+      if (ks > 1) part[q] = std::max(part[q], sizeof(T) * (size_t)ks * kk * nc);
+    };
+    const int pq = look ? 1 : 0;
+    std::function<void(int, int)> phase_needs = [&](int i, int w) {
+      if (w <= nb || (block && cqr_block_groups(m - i, w, std::min(256, partition ? pcus : h->num_cus)) > 0)) return;
+      const int w1 = split_of(w), w2 = w - w1;
+      phase_needs(i, w1);
+      product(pq, m - i, w2, w1);
+      phase_needs(i + w1, w2);
+      const int ks = std::max(1, std::min(32, (m - i - w1) / 256));
+      part[pq] = std::max(part[pq], sizeof(T) * (size_t)ks * w1 * w2);
+    };
+    for (int b = 0; b < nob; ++b) {
+      const int rows = m - bstart[b], c0 = bstart[b + 1], wn = (look && b + 1 < nob) ? bw(b + 1) : 0;
+      phase_needs(bstart[b], bw(b));
+      product(1, rows, wn, bw(b));
+      product(0, rows, n - c0 - wn, bw(b));
+      product(0, rows, nrhs, bw(b));
+    }
+    const size_t vbytes = sizeof(T) * (size_t)m * nbo, tbytes = sizeof(T) * (size_t)nbo * nbo;
+    const std::pair<Buffer*, size_t> need[] = {
+        {&h->vbuf, vbytes},
+        {&h->tbuf, tbytes},
+        {&h->vbuf2, look ? vbytes : 0},
+        {&h->tbuf2, look ? tbytes : 0},
+        {&h->gram, sizeof(T) * (size_t)nb * nb},
+        {&h->ppart, sizeof(T) * 2 * (size_t)kMaxPanelGroups * nb + 64},
+        {&h->rowbuf, sizeof(T) * 2 * (size_t)nb},
+        {&h->sync, sizeof(unsigned) * (size_t)sync_words},
+        {&h->cqr_part, block ? std::max(part_b, sizeof(double) * (size_t)std::max(3, (m + 63) / 64) * kCqrBlockPart) : part_b},
+        {&h->cqr_gsum, block ? std::max(gsum_b, sizeof(double) * kCqrBlockGrams * kCqrBlockPart) : gsum_b},
+        {&h->cqr_scratch, block ? std::max(scratch_b, sizeof(double) * kCqrBlockScratch) : scratch_b},
+        {&h->misc2, misc2_bytes},
+        {&h->wbuf, wz[0]},
+        {&h->zbuf, wz[0]},
+        {&h->part, part[0]},
+        {&h->wbuf2, wz[1]},
+        {&h->zbuf2, wz[1]},
+        {&h->part2, part[1]},
+        {&h->exsave, split_scan ? sizeof(T) * (size_t)m * w0 : 0}};
+    return reserve(h, need, sizeof(need) / sizeof(need[0]));
+  };
+  if (use_block) {
+    int s = reserve_all(true);
+    if (s == RNPX_ERR_NOMEM) {
+      use_block = false;
+      (void)h->give_back_block();
+      s = reserve_all(false);
+    }
+    if (s) return s;
+  }
+  struct BlockBusy {
+    Handle* h;
+    ~BlockBusy() { h->block_busy = false; }
+  } block_busy{h};
+  h->block_busy = true;
   Buffer* vb[2] = {&h->vbuf, &h->vbuf2};
   Buffer* tb[2] = {&h->tbuf, &h->tbuf2};
   for (int q = 0; q < (look ? 2 : 1); ++q) {
@@ -691,41 +814,16 @@ int geqrf_dev(Handle* h, int m, int n, T* A, long lda, T* tau, T* B, int nrhs, l
   RNPX_TRY(h->gram.ensure(sizeof(T) * (size_t)nb * nb, h));
   RNPX_TRY(h->ppart.ensure(sizeof(T) * 2 * (size_t)kMaxPanelGroups * nb + 64, h));
   RNPX_TRY(h->rowbuf.ensure(sizeof(T) * 2 * (size_t)nb, h));
-  // (one panel's words more: a last block of one panel still uses two)
-  const int sync_words = 1 + 2 * npan + kCqrSyncWords * (npan + 1);
   RNPX_TRY(h->sync.ensure(sizeof(unsigned) * (size_t)sync_words, h));
-  // Outer blocks in one launch (real, 64-column panels, 128-column blocks,
-  // tuning panel 0): buffers for the block kernel (without room for them in the
-  // handle's budget: panel by panel).
-  bool use_block = !S<T>::cplx && h->tune.panel == 0 && nb == 64 && nbo % (2 * nb) == 0 &&
-                         cqr_block_groups(m, std::min(nb, k), std::min(256, h->num_cus)) > 0;
-  static_assert(2 * kCqrSyncWords >= kCqrBlockSyncWords, "a block uses its two panels' sync words");
-  if (use_block) {
-    const std::pair<Buffer*, size_t> need[] = {
-        {&h->cqr_part, sizeof(double) * (size_t)std::max(3, (m + 63) / 64) * kCqrBlockPart},
-        {&h->cqr_gsum, sizeof(double) * kCqrBlockGrams * kCqrBlockPart},
-        {&h->cqr_scratch, sizeof(double) * kCqrBlockScratch}};
-    const int s = reserve(h, need, 3);
-    if (s == RNPX_ERR_NOMEM) use_block = false;
-    else if (s) return s;
-  }
-  {
-    int g0 = 0, rw0 = 0;
-    if (use_cqr<T>(h, m, std::min(nb, k), nb, &g0, &rw0)) {
-      // later panels may use more (smaller) workgroups than the first
-      RNPX_TRY(h->cqr_part.ensure(sizeof(double) * (size_t)std::min(kCqrMaxGroups, h->num_cus) * 2560, h));
-      RNPX_TRY(h->cqr_gsum.ensure(sizeof(double) * (2 + 16) * 2560, h));  // gsum, then group sums
-      RNPX_TRY(h->cqr_scratch.ensure(sizeof(double) * kCqrScratch, h));
-    }
-  }
-  RNPX_TRY(h->misc2.ensure(sizeof(T) * (size_t)std::max(3 * nb * nb, 2 * (nbo / 2) * (nbo / 2)), h));
+  RNPX_TRY(h->cqr_part.ensure(part_b, h));
+  RNPX_TRY(h->cqr_gsum.ensure(gsum_b, h));
+  RNPX_TRY(h->cqr_scratch.ensure(scratch_b, h));
+  RNPX_TRY(h->misc2.ensure(misc2_bytes, h));
   RNPX_TRY(launch_zero_u32((unsigned*)h->sync.p, sync_words, st));
-  // An outer block of w columns is split into w1 = 2 nb (a block-kernel
-  // unit) or nb columns and the rest.  The parts of the merged V and T no
+  // The parts of the merged V and T no
   // panel writes -- V's rows above the second part, T's block below the
   // diagonal -- are zero; they are cleared once, for the full width and the
   // last block's, in both buffers.
-  auto split_of = [&](int w) { return w > 2 * nb ? 2 * nb : nb; };
   std::function<int(int, long, T*, T*)> zero_parts = [&](int w, long off, T* Vq, T* Tq) -> int {
     if (w <= nb) return RNPX_OK;
     const int w1 = split_of(w), w2 = w - w1;
@@ -858,15 +956,7 @@ int geqrf_dev(Handle* h, int m, int n, T* A, long lda, T* tau, T* B, int nrhs, l
   hipStream_t ps = h->pstream, us = st;
   // CU partition: every panel kernel of this call must fit the panel set
   // (their workgroups meet at grid-wide reductions).
-  int pcus = h->tune.panel_cus;
-  if (pcus == 0) {
-    static const int env_cus = [] {
-      const char* e = getenv("RNPX_PANEL_CUS");
-      return e ? atoi(e) : 0;
-    }();
-    pcus = env_cus;
-  }
-  if (pcus > 0 && G0 <= pcus && !h->ext_pstream && h->ensure_partition(pcus) > 0) {
+  if (partition && h->ensure_partition(pcus) > 0) {
     ps = h->part_ps;
     us = h->part_us;
     h->panel_cap = pcus;

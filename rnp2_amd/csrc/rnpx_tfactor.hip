@@ -142,22 +142,22 @@ __global__ void gram_sum_blocks_kernel(int k, int w, int ns, const T* __restrict
   gram[b * ws + e] = s;
 }
 
-int gram_blocks_slices(int n, int k, int w, int* kslice) {
+int gram_blocks_slices(int n, int k, int w, int most, int* kslice) {
   const int nblk = (k + w - 1) / w, tiles = (w <= 64 ? 1 : 4) * nblk;
   // about three workgroups per CU in all, slices of at least 32 rows (16 rows
   // of a slice take about a microsecond, whatever else is idle) and at most
-  // 96 of them (their sum takes about half a microsecond for eight)
-  int ns = std::max(1, std::min({96, n / 32, 768 / tiles}));
+  // `most` of them (their sum takes about half a microsecond for eight)
+  int ns = std::max(1, std::min({most, n / 32, 768 / tiles}));
   *kslice = ((n + ns - 1) / ns + 15) / 16 * 16;
   return (n + *kslice - 1) / *kslice;
 }
 
 template <typename T>
-hipError_t launch_gram_blocks(int n, int k, int w, const T* V, long ldv, const T* tau, T* gram, T* part,
+hipError_t launch_gram_blocks(int n, int k, int w, int most, const T* V, long ldv, const T* tau, T* gram, T* part,
                               hipStream_t st) {
   if (k < 1 || n < k || ldv < n) return hipErrorInvalidValue;
   int kslice = 0;
-  const int ns = gram_blocks_slices(n, k, w, &kslice), full = k / w, rest = k - full * w;
+  const int ns = gram_blocks_slices(n, k, w, most, &kslice), full = k / w, rest = k - full * w;
   const size_t ws = (size_t)w * w;
   const int nblk = full + (rest > 0), wlast = rest > 0 ? rest : w;
   if constexpr (S<T>::cplx)
@@ -172,7 +172,7 @@ hipError_t launch_gram_blocks(int n, int k, int w, const T* V, long ldv, const T
 #define RNPX_TF_INST(T)                                                                                       \
   template hipError_t launch_tfactor<T>(const T*, int, int, int, T*, int, hipStream_t, const unsigned*);      \
   template hipError_t launch_tfactor_blocks<T>(const T*, int, int, T*, hipStream_t);                          \
-  template hipError_t launch_gram_blocks<T>(int, int, int, const T*, long, const T*, T*, T*, hipStream_t);
+  template hipError_t launch_gram_blocks<T>(int, int, int, int, const T*, long, const T*, T*, T*, hipStream_t);
 RNPX_TF_INST(double)
 RNPX_TF_INST(zd)
 #undef RNPX_TF_INST
