@@ -20,6 +20,7 @@
 // refinement does not reach the tolerance (ill-conditioned A).
 // Each request's result depends only on its own data: the same bits alone or
 // in any mix.
+#include "rnpx_hostblocks.hpp"
 #include "rnpx_internal.hpp"
 
 #include <algorithm>
@@ -64,81 +65,19 @@ static double now_s() {
   return duration<double>(steady_clock::now().time_since_epoch()).count();
 }
 
-// Host memory for the requests' copies of A and B: pinned blocks that go back
-// to the server's list when a request is done, so that a submit neither faults
-// fresh pages in nor clears them before the copy (submitting a burst of 24
-// requests, 340 MB, took 63 ms that way and takes 9 now; the burst 74.5 -> 45.2
-// ms), and the worker's transfer to the device is one asynchronous DMA.  At
-// most kPinnedBytes in all, in use or idle, given back when the server is
-// destroyed; a request beyond that (or where pinned memory is refused) takes
-// ordinary memory.
-struct HostBlock {
-  double* p = nullptr;
-  size_t bytes = 0;
-  bool pinned = false;
+struct HipPin {
+  static bool pin(void** p, size_t bytes) {
+    if (hipHostMalloc(p, bytes, hipHostMallocPortable) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+  }
+  static void unpin(void* p) { (void)hipHostFree(p); }
 };
-class HostBlocks {
- public:
-  ~HostBlocks() {
-    for (HostBlock& b : idle_) hipHostFree(b.p);
-  }
-  HostBlock take(size_t bytes) {
-    // sizes in eighths of a power of two, 64 KB at least: a block serves
-    // requests down to half its size
-    size_t unit = (size_t)64 << 10;
-    while (unit * 16 < bytes) unit *= 2;
-    const size_t want = std::max<size_t>((size_t)64 << 10, (bytes + unit - 1) / unit * unit);
-    std::vector<HostBlock> drop;
-    bool room = false;
-    {
-      std::lock_guard<std::mutex> lk(mu_);
-      size_t best = idle_.size();
-      for (size_t i = 0; i < idle_.size(); ++i)
-        if (idle_[i].bytes >= want && idle_[i].bytes <= 2 * want &&
-            (best == idle_.size() || idle_[i].bytes < idle_[best].bytes))
-          best = i;
-      if (best < idle_.size()) {
-        HostBlock b = idle_[best];
-        idle_.erase(idle_.begin() + (long)best);
-        return b;
-      }
-      // room for a new one, if need be in place of idle blocks of other sizes
-      while (!idle_.empty() && held_ + want > kPinnedBytes) {
-        held_ -= idle_.back().bytes;
-        drop.push_back(idle_.back());
-        idle_.pop_back();
-      }
-      room = held_ + want <= kPinnedBytes;
-      if (room) held_ += want;
-    }
-    // (the driver's calls, tens of milliseconds for a large block, outside the lock)
-    for (HostBlock& b : drop) hipHostFree(b.p);
-    if (room) {
-      HostBlock b{nullptr, want, true};
-      if (hipHostMalloc((void**)&b.p, want, hipHostMallocPortable) == hipSuccess) return b;
-      (void)hipGetLastError();
-      std::lock_guard<std::mutex> lk(mu_);
-      held_ -= want;
-    }
-    return HostBlock{static_cast<double*>(std::malloc(std::max<size_t>(bytes, 8))), bytes, false};
-  }
-  void give(HostBlock& b) {
-    if (!b.p) return;
-    if (b.pinned) {
-      std::lock_guard<std::mutex> lk(mu_);
-      idle_.push_back(b);
-    } else {
-      std::free(b.p);
-    }
-    b = HostBlock{};
-  }
-
- private:
-  static constexpr size_t kPinnedBytes = (size_t)1 << 30;
-  std::mutex mu_;
-  std::vector<HostBlock> idle_;
-  size_t held_ = 0;
-};
+// The requests' copies of A and B.  A burst of 24 requests, 340 MB, takes 45 ms
+// with them (74 in memory allocated and cleared for each request); the first burst
+// of a server, or after a pause, pins its blocks and takes 65 to 70.
+constexpr size_t kPinnedBytes = (size_t)1 << 30;
+constexpr std::chrono::seconds kPinnedIdle(10);  // after that long without a request the idle blocks go back
 
 struct Request {
   long long id = 0;
@@ -160,7 +99,7 @@ struct Server {
   std::vector<std::thread> workers;
   std::vector<Handle*> handles;
   hipStream_t panel_stream = nullptr;
-  HostBlocks blocks;
+  HostBlocks<HipPin> blocks{kPinnedBytes};
   size_t in_use = 0;
   long long next_id = 1;
   int bypassed = 0;
@@ -324,11 +263,19 @@ static void worker_main(Server* s, int w) {
     work.clear();
     {
       std::unique_lock<std::mutex> lk(s->mu);
-      s->cv.wait(lk, [&] {
+      auto ready = [&] {
         if (s->stop) return true;
         take_work(s, work);
         return !work.empty();
-      });
+      };
+      if (!s->cv.wait_for(lk, kPinnedIdle, ready)) {
+        if (s->queue.empty() && s->in_use == 0) {
+          lk.unlock();
+          s->blocks.trim();
+          lk.lock();
+        }
+        s->cv.wait(lk, ready);
+      }
       if (work.empty() && s->stop) break;
       const double t = now_s();
       for (Request* r : work) {
@@ -416,7 +363,8 @@ int rnpx_server_submit(rnpx_server srv, size_t m, size_t n, size_t nrhs, const d
   r->bytes = footprint(r->m, r->n, r->nrhs, s->cfg.mode);
   const bool too_large = s->cfg.hbm_budget && r->bytes > s->cfg.hbm_budget;
   if (!too_large) {
-    r->mem = s->blocks.take(sizeof(double) * (m * n + m * nrhs));
+    // (a small request is gathered into a batch on the host, never transferred from here)
+    r->mem = s->blocks.take(sizeof(double) * (m * n + m * nrhs), m > (size_t)kSmallM);
     if (!r->mem.p) {
       delete r;
       return RNPX_ERR_NOMEM;
