@@ -481,8 +481,9 @@ struct WyPlan {
   int w, chunk;
 };
 
-// The widest plan that the device holds: every block's T at once (MultQ: at
-// most 2048 columns, whose V copy it also keeps), else one block at a time,
+// The widest plan that the device holds: every block's T at once (MultQ: as many
+// columns as kWyCopy bytes of V, of which it keeps a copy, at most 2048), else one
+// block at a time,
 // down to the 64 (complex 32) columns that need least -- which a handle with a
 // memory budget always takes, so that its budget is left to other calls.  own_v:
 // V lives in vbuf, chunk columns of it (MultQ); rows, cols: the matrix each
@@ -491,12 +492,14 @@ struct WyPlan {
 // the T factors formed at once take 70 us per 64 columns off the chain of
 // blocks: MultQ of a 6001 x 1999 matrix by 1500 reflectors went from 5.06 to
 // 2.21 ms, GenerateQ of 8192 x 2048 from 5.77 to 2.31 ms.
+constexpr size_t kWyCopy = (size_t)256 << 20;  // a thousandth of the device's memory
 template <typename T>
 static int wy_plan(Handle* h, bool own_v, bool left, int nq, int k, int rows, int cols, bool shrink, WyPlan* out) {
   // no wider than the reflectors: a T leaf of 64 complex columns takes 30 us where
   // one of 32 takes 15
   const int wide = S<T>::cplx ? (k > 32 ? 64 : 32) : (k > 64 ? 128 : 64), narrow = pick_nb<T>(h, rows, cols);
-  const int most = own_v ? std::min(k, 2048) : k;
+  const int fit = (int)std::min<size_t>(2048, kWyCopy / (sizeof(T) * (size_t)nq)) / wide * wide;
+  const int most = own_v ? std::min(k, std::max(wide, fit)) : k;
   const WyPlan tries[3] = {{wide, (most + wide - 1) / wide * wide}, {wide, wide}, {narrow, narrow}};
   for (int t = h->budget ? 2 : 0; t < 3; ++t) {
     const WyPlan& p = tries[t];

@@ -72,3 +72,24 @@ def test_generateq_plan_edges(dt, m, n, k, budget):
         assert float((A.cpu() - want).norm()) <= 10 * max(k, 1) * EPS * n ** 0.5
     finally:
         h.close()
+
+
+@pytest.mark.parametrize("dt,q,k", [(torch.float64, 32768, 1500), (torch.complex128, 20000, 1000)])
+def test_multq_copy_of_v_is_bounded(dt, q, k):
+    """256 MB of V at a time, whatever the number of reflectors: chunks of 1024
+    and 832 columns here, in both directions."""
+    a, tau = stored(q, k, dt, q + k)
+    A, tau = dev(a), tau.cuda()
+    C = dev(torch.randn(q, 5, dtype=dt, generator=torch.Generator().manual_seed(1)))
+    C0 = C.clone()
+    torch.cuda.synchronize()
+    h = R.Handle()
+    try:
+        h.ormqr("L", "C", A, tau, C)
+        h.ormqr("L", "N", A, tau, C)
+        h.synchronize()
+        assert float((C - C0).norm()) <= 20 * k * EPS * float(C0.norm())
+        vbuf = 256 << 20
+        assert h.workspace_bytes() <= vbuf + vbuf // 8 + (64 << 20)  # V with its headroom; Grams, T, partial sums
+    finally:
+        h.close()
