@@ -39,19 +39,11 @@ __device__ __forceinline__ bool better(double va, int ia, double vb, int ib) {
   return (va > vb) || (va == vb && ia < ib);
 }
 
-template <typename T>
-__device__ __forceinline__ T ld_part(const double* p) {
-  if constexpr (S<T>::cplx) return mkz(p[0], p[1]);
-  else return p[0];
-}
-template <typename T>
-__device__ __forceinline__ void st_part(double* p, T v) {
-  if constexpr (S<T>::cplx) {
-    p[0] = v.x;
-    p[1] = v.y;
-  } else {
-    p[0] = v;
-  }
+// A complex entry in the panel's scratch.
+__device__ __forceinline__ zd ld_part(const double* p) { return mkz(p[0], p[1]); }
+__device__ __forceinline__ void st_part(double* p, zd v) {
+  p[0] = v.x;
+  p[1] = v.y;
 }
 
 }  // namespace
@@ -349,9 +341,10 @@ __global__ __launch_bounds__(kLuRowThreads) void lu_row_panel_kernel(LuPanelArgs
 // row, then the row's kLuNB entries), rowc[2][2*kLuNB] (row c).
 constexpr int kLuSlot = 2 + 2 * kLuNB;
 
-template <typename T, int RW>
+template <int RW>
 __global__ __launch_bounds__(256) void lu_panel_kernel(LuPanelArgs a) {
-  constexpr int NB = kLuNB, LDS_S = NB + 1, TE = S<T>::cplx ? 2 : 1;
+  using T = zd;
+  constexpr int NB = kLuNB, LDS_S = NB + 1;
   __shared__ T Sl[RW][LDS_S];
   __shared__ T ubuf[NB], ocbuf[NB];
   __shared__ double redv[4];
@@ -421,9 +414,9 @@ __global__ __launch_bounds__(256) void lu_panel_kernel(LuPanelArgs a) {
       my[1] = (double)bi;
     }
     if (bi != 0x7fffffff)
-      for (int q = tid; q < NB; q += 256) st_part<T>(my + 2 + TE * q, Sl[bi - gr0][q]);
+      for (int q = tid; q < NB; q += 256) st_part(my + 2 + 2 * q, Sl[bi - gr0][q]);
     if (c >= gr0 && c < gr0 + RW)
-      for (int q = tid; q < NB; q += 256) st_part<T>(rowc + TE * q, Sl[c - gr0][q]);
+      for (int q = tid; q < NB; q += 256) st_part(rowc + 2 * q, Sl[c - gr0][q]);
     // every workgroup waits for all the candidates, then reduces them in
     // workgroup order itself (no second hand-off)
     unsigned* cnt = a.sync + 2 * c;
@@ -448,7 +441,7 @@ __global__ __launch_bounds__(256) void lu_panel_kernel(LuPanelArgs a) {
     // candidates' (one round trip fewer per column).
     static_assert(NB <= 256, "a thread per entry of row c");
     T ocv = zero;
-    if (tid < NB) ocv = ld_part<T>(rowc + TE * tid);
+    if (tid < NB) ocv = ld_part(rowc + 2 * tid);
     {
       double v = -2.0;
       int i = 0x7fffffff, w = -1;
@@ -503,7 +496,7 @@ __global__ __launch_bounds__(256) void lu_panel_kernel(LuPanelArgs a) {
     }
     const int p = pw[0], w = pw[1];
     // 3. pivot row u: the winner's row, or row c itself (already in ocbuf)
-    if (tid < NB) ubuf[tid] = (w >= 0) ? ld_part<T>(part + (size_t)w * kLuSlot + 2 + TE * tid) : ocbuf[tid];
+    if (tid < NB) ubuf[tid] = (w >= 0) ? ld_part(part + (size_t)w * kLuSlot + 2 + 2 * tid) : ocbuf[tid];
     __syncthreads();
     if (c >= gr0 && c < gr0 + RW)
       for (int q = tid; q < NB; q += 256) Sl[c - gr0][q] = ubuf[q];
@@ -665,8 +658,8 @@ hipError_t launch_lu_axpy(int n, const T* x, T* y, hipStream_t st) {
 int lu_panel_rows(int mp, int max_groups, int cplx) {
   // Real: 512 rows per workgroup (at most 128 workgroups offer a candidate).
   if (!cplx) return mp <= 256 * max_groups && mp <= 128 * kLuRowThreads ? kLuRowThreads : 0;
-  // Complex: 128-row blocks (64 measured 72.4 ms against 69.9 on a real
-  // 8192^2 with this kernel); RNPX_LU_PANEL_RW overrides.
+  // Complex: 128-row blocks; RNPX_LU_PANEL_RW (64 or 128) overrides, for
+  // complex panels only.
   static const int pref = [] {
     const char* e = getenv("RNPX_LU_PANEL_RW");
     return e ? atoi(e) : 0;
@@ -687,8 +680,8 @@ hipError_t launch_lu_panel(const LuPanelArgs& a, int rw, hipStream_t st) {
     hipLaunchKernelGGL(lu_row_panel_kernel, dim3(G), dim3(kLuRowThreads), 0, st, a);
   } else {
     if (!a.sync || !a.part || !a.rowc) return hipErrorInvalidValue;
-    if (rw == 64) hipLaunchKernelGGL((lu_panel_kernel<T, 64>), dim3(G), dim3(256), 0, st, a);
-    else if (rw == 128) hipLaunchKernelGGL((lu_panel_kernel<T, 128>), dim3(G), dim3(256), 0, st, a);
+    if (rw == 64) hipLaunchKernelGGL((lu_panel_kernel<64>), dim3(G), dim3(256), 0, st, a);
+    else if (rw == 128) hipLaunchKernelGGL((lu_panel_kernel<128>), dim3(G), dim3(256), 0, st, a);
     else return hipErrorInvalidValue;
   }
   return hipGetLastError();
