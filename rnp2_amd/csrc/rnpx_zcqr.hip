@@ -188,7 +188,7 @@ __device__ __forceinline__ void rotate4(ZCol& a) {
 // Upper Cholesky factor R (left lanes, rows <= c) and R^{-H} (right lanes) of
 // [G | I]; dg: G(c, c).  False (uniformly) on a pivot below rel * its diagonal or
 // not finite.
-__device__ __forceinline__ bool chol_wave(ZCol& a, double dg, double rel) {
+__device__ __forceinline__ bool chol_wave(ZCol& a, double dg, double rel, int lane) {
   bool ok = true;
 #pragma unroll 1
   for (int b = 0; b < NB / 4; ++b) {
@@ -199,6 +199,7 @@ __device__ __forceinline__ bool chol_wave(ZCol& a, double dg, double rel) {
       ok = ok && d > rel * readlane_t(dg, j) && isfinite(d);
       const double inv = small64::rsq_nr(d);
       a.w[s] = a.w[s] * inv;  // R(j, c), c >= j
+      if (lane == j) a.w[s].y = 0.0;  // the diagonal is real; G's has a rounding error there
 #pragma unroll
       for (int q = 0; q < NB / 4; ++q)
         if (q < NB / 4 - b) {
@@ -238,7 +239,7 @@ __global__ __launch_bounds__(64) void chol_kernel(const zd* __restrict__ G, zd* 
   }
   bad = bad || !(dg >= 0x1p-600 && dg <= 0x1p600);
   bool ok = __ballot(bad) == 0;
-  if (ok) ok = chol_wave(a, dg, 0x1p-40);
+  if (ok) ok = chol_wave(a, dg, 0x1p-40, lane);
   if (!ok) {
     if (lane == 0) *fail = 1u;
     return;

@@ -81,3 +81,13 @@ def test_rejected_panels(kind):
         assert qr_residual(a, q, np.triu(af[:n])) <= 10 and orth_error(q) <= 10
     else:
         check(a, af, tau, kind)
+
+
+@pytest.mark.parametrize("m,n", [(100, 64), (300, 96), (2000, 500), (4096, 1024)])
+def test_diagonal_of_r_is_real(m, n):
+    """Generate's beta is real (Reflector.hpp:131, 150): no rounding error is left
+    in R's diagonal's imaginary parts, whichever panel made it."""
+    rng = np.random.default_rng(m)
+    a = rng.standard_normal((m, n)) + 1j * rng.standard_normal((m, n))
+    af, _ = R.factor(a)
+    assert np.array_equal(np.diag(af).imag, np.zeros(n))
