@@ -522,13 +522,12 @@ __global__ __launch_bounds__(256) void cqr_panel_kernel(CqrArgs a) {
 // in the halves named by zero_tails such a running pivot (within 2^-40 of one)
 // rejects the block.
 // Bound by the chain of two grid reductions, two Cholesky and two LU
-// factorizations of 64 x 64.  Against two 64-column panels joined inside the
-// launch (six reductions, the second panel's Gram after the first one's
-// reconstruction; 370 KB of unrolled code where this is 96 KB, most of it cold in
-// the instruction cache): 201 -> 168 us per block at 1931 rows and below; the
-// factorization of 1931 x 1207, whose last 55 columns also run here now,
-// 2.70 -> 2.24 ms, 8192^2 29.4 -> 27.1 ms, 250 x 64 0.11 ms as before,
-// 100 x 64 0.32 -> 0.11 ms, 100 x 100 0.55 -> 0.27 ms.
+// factorizations of 64 x 64: 168 us per block at 1931 rows and below, 275 at
+// 16384; 1931 x 1207 factors in 2.18 ms, 8192^2 in 26.4, 100 x 100 in 0.24.  Two
+// 64-column panels joined inside the launch (six reductions, the second panel's
+// Gram after the first one's reconstruction; 370 KB of unrolled code where this is
+// 96 KB, most of it cold in the instruction cache) and ragged ends column by
+// column take 201 us, 2.70, 29.4 and 0.55 ms.
 // ---------------------------------------------------------------------------
 namespace {
 
@@ -603,9 +602,9 @@ __device__ __forceinline__ void grid_step(const CqrBlockArgs& a, int step, int g
 // sums its slice of the entries over the partials in a fixed order (so the result
 // does not depend on timing) and stores it; the sum is complete at the second
 // grid-wide step.  red: 512 doubles of LDS scratch.  With counters and agent-scope
-// releases a reduction took 10 us at 64 workgroups, 21 at 128 and 38 at 256; with
+// releases a reduction takes 10 us at 64 workgroups, 21 at 128 and 38 at 256; with
 // marks and stores written through the 256-workgroup block (16384 rows) is 28 us
-// faster in all, least squares 16384 x 2048 8.92 -> 8.46 ms.
+// faster in all (least squares 16384 x 2048: 8.46 ms against 8.92).
 __device__ __forceinline__ void blk_allreduce(const CqrBlockArgs& a, int elems, int pass, int g, int G, double* gs,
                                               double* red, int tid) {
   grid_step(a, 2 * pass + 1, g, G, tid);

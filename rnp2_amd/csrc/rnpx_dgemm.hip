@@ -72,11 +72,11 @@ struct Op {
   // outside it is some other entry.  Outside rows (rows of op(A) or columns of
   // op(B)) only feed outputs that are never stored; outside K is zeroed by
   // store().  VEC: one 16-byte load per pair, of 8-byte alignment (global
-  // loads need no more, so any leading dimension and base takes it; against two
-  // 8-byte loads at an odd leading dimension, a 128 x 1079 by 1931 product
-  // went from 119 to 110 us, the aligned one staying at 108); needs two entries along the pairs.  The pair that would
-  // cross an odd extent is read one entry earlier; store() takes its second
-  // entry for the first (here it would wait for the loads).
+  // loads need no more, so any leading dimension and base takes it: a 128 x 1079
+  // by 1931 product with odd leading dimensions takes 110 us, with two 8-byte
+  // loads a pair 119, aligned 108); needs two entries along the pairs.  The pair
+  // that would cross an odd extent is read one entry earlier; store() takes its
+  // second entry for the first (here it would wait for the loads).
   template <bool VEC>
   __device__ static inline void fetch(double2 (&v)[NV], const double* __restrict__ p, long ld, int r0, int k0,
                                       int rlim, int klim, int tid) {

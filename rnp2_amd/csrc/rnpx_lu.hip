@@ -161,8 +161,8 @@ __device__ __forceinline__ Word get_word(const Word* p) {
 // reads every workgroup's offer, then the winner's row.
 // Bound by that hand-off's latency: 3.5 us per column at 8192 rows on 16
 // workgroups, against 7.2 us for rows in LDS on 64 workgroups with row swaps, a
-// counter, and a release and acquire per column; 8192^2 with the solve of 16
-// right-hand sides 76.1 -> 40.9 ms together with the list of moved rows below.
+// counter, and a release and acquire per column.  With the list of moved rows
+// below, 8192^2 and the solve of 16 right-hand sides take 37 ms.
 __global__ __launch_bounds__(kLuRowThreads) void lu_row_panel_kernel(LuPanelArgs a) {
   constexpr int NB = kLuNB, NW = kLuRowThreads / 64;
   __shared__ double wv[NW], urow[NB], uw[NW][NB];

@@ -483,15 +483,15 @@ struct WyPlan {
 
 // The widest plan that the device holds: every block's T at once (MultQ: as many
 // columns as kWyCopy bytes of V, of which it keeps a copy, at most 2048), else one
-// block at a time,
-// down to the 64 (complex 32) columns that need least -- which a handle with a
-// memory budget always takes, so that its budget is left to other calls.  own_v:
-// V lives in vbuf, chunk columns of it (MultQ); rows, cols: the matrix each
-// block is applied to, block at column i touching rows and columns as in the
-// callers below.  128-column (complex 64) blocks halve the passes over C, and
-// the T factors formed at once take 70 us per 64 columns off the chain of
-// blocks: MultQ of a 6001 x 1999 matrix by 1500 reflectors went from 5.06 to
-// 2.21 ms, GenerateQ of 8192 x 2048 from 5.77 to 2.31 ms.
+// block at a time, down to the tuned panel width (64, complex 32), which needs
+// least -- and which a handle with a memory budget always takes, so that its
+// budget is left to other calls.  own_v: V lives in vbuf, chunk columns of it
+// (MultQ); rows, cols: the matrix each block is applied to, block at column i
+// touching rows and columns as in the callers below.  128-column (complex 64)
+// blocks halve the passes over C, and the T factors formed at once take 70 us per
+// 64 columns off the chain of blocks: MultQ of a 6001 x 1999 matrix by 1500
+// reflectors takes 2.19 ms, GenerateQ of 8192 x 2048 2.31; 64 columns and a T at a
+// time 5.06 and 5.77.
 constexpr size_t kWyCopy = (size_t)256 << 20;  // a thousandth of the device's memory
 template <typename T>
 static int wy_plan(Handle* h, bool own_v, bool left, int nq, int k, int rows, int cols, bool shrink, WyPlan* out) {
@@ -823,10 +823,9 @@ int geqrf_dev(Handle* h, int m, int n, T* A, long lda, T* tau, T* B, int nrhs, l
   RNPX_TRY(h->cqr_scratch.ensure(scratch_b, h));
   RNPX_TRY(h->misc2.ensure(misc2_bytes, h));
   RNPX_TRY(launch_zero_u32((unsigned*)h->sync.p, sync_words, st));
-  // The parts of the merged V and T no
-  // panel writes -- V's rows above the second part, T's block below the
-  // diagonal -- are zero; they are cleared once, for the full width and the
-  // last block's, in both buffers.
+  // The parts of the merged V and T no panel writes -- V's rows above the
+  // second part, T's block below the diagonal -- are zero; they are cleared
+  // once, for the full width and the last block's, in both buffers.
   std::function<int(int, long, T*, T*)> zero_parts = [&](int w, long off, T* Vq, T* Tq) -> int {
     if (w <= nb) return RNPX_OK;
     const int w1 = split_of(w), w2 = w - w1;

@@ -27,9 +27,9 @@
 // quotients.  Nothing else is on it: R_pq is loaded before the flag is polled,
 // x goes without fences, and with four right-hand sides to a workgroup every
 // workgroup of n = 8192, 16 right-hand sides is resident at once and R is read a
-// quarter as often.  That solve: 2650 us with one right-hand side to a workgroup,
-// R loaded after the flag and an agent-scope fence on each side; 920 us now
-// (7.2 us a block).
+// quarter as often.  That solve takes 920 us (7.2 us a block), with one right-hand
+// side to a workgroup, R loaded after the flag and an agent-scope fence on each
+// side 2650.
 #include "rnpx_kernels.hpp"
 
 namespace rnpx {

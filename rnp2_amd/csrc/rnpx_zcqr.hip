@@ -218,11 +218,11 @@ __device__ __forceinline__ bool chol_wave(ZCol& a, double dg, double rel, int la
 }
 
 // Pass 1: R1 = chol(G1) and R1^{-1}, or the fail flag; one wave, since the kernel
-// is one serial chain: 25 us, 32 with a barrier, a square root and a division per
-// step over four waves and a substitution for the inverse.  0.6 us a step, the
-// row updates' v_readlanes and the branches between them.  (The reconstruction's
-// LU the same way took that kernel from 44 to 46 us: its steps already overlapped
-// the division with the row updates, which one wave does alone.)
+// is one serial chain: 25 us, against 32 with a barrier, a square root and a
+// division per step over four waves and a substitution for the inverse.  0.6 us a
+// step, the row updates' v_readlanes and the branches between them.  (With the
+// reconstruction's LU the same way that kernel takes 46 us instead of 44: over
+// four waves its steps overlap the division with the row updates.)
 __global__ __launch_bounds__(64) void chol_kernel(const zd* __restrict__ G, zd* __restrict__ R1,
                                                   zd* __restrict__ R1i, unsigned* fail) {
   const int lane = threadIdx.x, c = lane & 31;
