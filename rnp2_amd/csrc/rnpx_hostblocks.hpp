@@ -1,13 +1,45 @@
-// rnpx_hostblocks.hpp -- host memory for the server's copies of its requests.
-// Plain C++ over a pair of pin/unpin functions: a CPU test compiles this file.
+// rnpx_hostblocks.hpp -- the server's copies of its requests and the host memory
+// that they are in.  Plain C++ over a pair of pin/unpin functions: a CPU test
+// compiles this file.
 #pragma once
 #include <algorithm>
 #include <cstddef>
 #include <cstdlib>
+#include <cstring>
 #include <mutex>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 namespace rnpx {
+
+// dst (m x n, leading dimension m) = src (leading dimension lds): large
+// matrices split over host threads by columns (one thread copies a few GB/s;
+// a 8192 x 4096 request is 268 MB; a thread's start is worth about 4 MB).  A
+// thread that the system refuses leaves its columns to this one: the caller is
+// a C entry, where nothing may be thrown.
+template <class Thread>
+void copy_columns(double* dst, const double* src, size_t m, size_t n, size_t lds) {
+  const size_t bytes = sizeof(double) * m * n;
+  const size_t hw = std::max(1u, std::thread::hardware_concurrency());
+  const size_t nt = std::min<size_t>({(size_t)8, hw, n, std::max<size_t>(1, bytes >> 22)});
+  const size_t per = (n + nt - 1) / nt;
+  auto part = [&](size_t q) {
+    for (size_t j = std::min(n, q * per); j < std::min(n, (q + 1) * per); ++j)
+      std::memcpy(dst + j * m, src + j * lds, sizeof(double) * m);
+  };
+  Thread th[8];
+  for (size_t q = 1; q < nt; ++q) {
+    try {
+      th[q] = Thread(part, q);
+    } catch (const std::system_error&) {
+      part(q);
+    }
+  }
+  part(0);
+  for (Thread& x : th)
+    if (x.joinable()) x.join();
+}
 
 struct HostBlock {
   double* p = nullptr;

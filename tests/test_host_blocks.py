@@ -1,7 +1,8 @@
 """The server's pinned request memory, with counting pin functions in a CPU
 build: the cap holds, idle blocks are dropped only where that makes room (the
 longest unused first), memory that no transfer reads is not pinned, trim() gives
-every idle block back, and several threads share the list."""
+every idle block back, and several threads share the list.  The copies into it are
+whole where the system refuses threads."""
 import os
 import shutil
 import subprocess
@@ -20,10 +21,38 @@ struct Fake {
   static bool pin(void** p, size_t n) { if (refuse) return false; ++pins; *p = std::malloc(n); return true; }
   static void unpin(void* p) { ++unpins; std::free(p); }
 };
+// a thread that cannot be had every other time
+struct Scarce : std::thread {
+  static int tries;
+  Scarce() = default;
+  Scarce(Scarce&&) = default;
+  Scarce& operator=(Scarce&&) = default;
+  template <class F> Scarce(F f, size_t q) : std::thread(start(), f, q) {}
+  struct Run { template <class F> void operator()(F f, size_t q) { f(q); } };
+  static Run start() {
+    if (++tries % 2) throw std::system_error(std::make_error_code(std::errc::resource_unavailable_try_again));
+    return Run();
+  }
+};
+int Scarce::tries = 0;
+template <class T> static bool copies(size_t m, size_t n, size_t lds) {
+  std::vector<double> a(lds * n), b(m * n, -1.0);
+  for (size_t i = 0; i < a.size(); ++i) a[i] = (double)i;
+  rnpx::copy_columns<T>(b.data(), a.data(), m, n, lds);
+  for (size_t j = 0; j < n; ++j)
+    for (size_t i = 0; i < m; ++i)
+      if (b[i + j * m] != a[i + j * lds]) return false;
+  return true;
+}
 #define CHECK(x) do { if (!(x)) { std::printf("line %d: %s (pins %d unpins %d)\n", __LINE__, #x, pins.load(), unpins.load()); return 1; } } while (0)
 int main() {
   using namespace rnpx;
   const size_t MB = 1 << 20;
+  for (size_t n : {1, 2, 7, 9, 1000, 5000}) {
+    CHECK(copies<std::thread>(1000, n, 1003));
+    CHECK(copies<Scarce>(1000, n, 1003));
+  }
+  CHECK(Scarce::tries > 3);
   {
     HostBlocks<Fake> h(100 * MB);
     HostBlock a = h.take(30 * MB, true), b = h.take(30 * MB, true), c = h.take(30 * MB, true);
