@@ -140,7 +140,7 @@ def test_lu_words_are_single_accesses(asm):
     assert sum("dwordx2" in s for s in loads) >= 5 * 8 and all(re.match(r"global_load_(dwordx2|dword)\b", s) for s in loads)
 
 
-def test_checker_flags_an_unwaited_mark():
+def test_an_unwaited_mark_is_seen():
     mark = r"global_store_byte\b.*sc1"
     data, wait, bar, byte = ("global_store_dwordx2 v[0:1], v[2:3], off sc1", "s_waitcnt vmcnt(0)", "s_barrier",
                              "global_store_byte v1, v0, s[4:5] sc1")
